@@ -148,6 +148,7 @@ int plan_forward(Handle* h, int B, int texH, int texW, const float* vpos, const 
   p.cams = h->cams.p; p.fnormal = h->fnormal.p; p.tris = h->tris.p; p.proj = h->proj.p;
   p.counters = h->counters.p; p.large = h->large.p; p.large_box = h->large_box;
   p.mesh_id = 0; p.shared_queue = false;
+  p.raster_items = (int64_t)B * h->C * h->F;
   p.tiled = tiled;
   p.tile_count = tiled ? h->tile_count.p : nullptr;
   p.bins = tiled ? h->bins.p : nullptr;

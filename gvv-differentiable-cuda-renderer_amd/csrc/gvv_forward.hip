@@ -180,6 +180,15 @@ __global__ void __launch_bounds__(256) k_vertices_multi(MeshTable<VertexArgs> t)
 }
 
 constexpr int kLargeWorkgroups = 4096;
+// (view, face) items up to which the depth pass gives 16, or 4, lanes to a face instead of one.
+// A wavefront's time is a serial chain over its faces' lines and candidates, so with fewer than
+// about 4096 wavefronts the chain, not the chip, is the kernel's time: 20,480 items (4 x 256^2
+// sphere) took 126 us with one lane and 15 us with 16 lanes to a face; 245,760 items
+// (12 views of 517 x 389) 131 against 87 us with 4.  Above the line the per-face setup that the
+// lanes of a face repeat costs more than it gains (96,000 items with 16 lanes: forward + backward
+// 181 against 171 us with 4).  The meshes of a multi-mesh run fill the chip together, so their
+// items count together (8 uneven meshes: 2.10 ms when each mesh chose by its own, 1.86 ms).
+constexpr int64_t kRasterItems16 = 65536, kRasterItems4 = 262144;
 
 struct RasterFace {
   int f, i0, i1, i2;
@@ -215,8 +224,8 @@ __device__ __forceinline__ void stage_face(FaceStage* dst, const TriSetup& t, fl
 }
 
 // Registers of the face a lane staged (its staging slot is that lane), read by the lanes that
-// test its candidates with a cross-lane permute.  The large-face pass holds its one face in
-// every lane.
+// test its candidates with a cross-lane permute (G lanes hold a face: the first is slot * G).
+// The large-face pass holds its one face in every lane.
 struct StageOwner {
   int f, bc, x0, y0, bw;
 };
@@ -241,6 +250,7 @@ __device__ __forceinline__ unsigned cand_word(bool packed, bool single, int slot
 // Each lane takes candidates lane, lane+64, ...; all lanes run the expensive test together.
 // `single`: the candidates of the large-face pass, which stages one face (slot 0).  Called in
 // wave-uniform control flow: the owner reads need every lane active.
+template <int G>
 __device__ __forceinline__ void flush_candidates(const FaceStage* st, const StageOwner& own, const unsigned* cand,
                                                  int count, const Camera* __restrict__ cams, bool one_view, int bc0,
                                                  unsigned long long* __restrict__ keys, int W, int H, bool single,
@@ -259,14 +269,14 @@ __device__ __forceinline__ void flush_candidates(const FaceStage* st, const Stag
     } else {
       slot = single ? 0 : (int)(c >> 24);
       const unsigned p = single ? c : (c & 0xffffffu);
-      const int x0 = __shfl(own.x0, slot, 64), y0 = __shfl(own.y0, slot, 64);
-      const unsigned w = (unsigned)__shfl(own.bw, slot, 64);
+      const int x0 = __shfl(own.x0, slot * G, 64), y0 = __shfl(own.y0, slot * G, 64);
+      const unsigned w = (unsigned)__shfl(own.bw, slot * G, 64);
       const unsigned dy = valid ? p / w : 0u;
       u = x0 + (int)(p - dy * w);
       v = y0 + (int)dy;
     }
-    const int f = __shfl(own.f, slot, 64);
-    const int bc = one_view ? bc0 : __shfl(own.bc, slot, 64);
+    const int f = __shfl(own.f, slot * G, 64);
+    const int bc = one_view ? bc0 : __shfl(own.bc, slot * G, 64);
     if (!valid) continue;
     const float4 q0 = st[slot].q[0], q1 = st[slot].q[1], q2 = st[slot].q[2], q3 = st[slot].q[3];
     const Camera& cam = cams[bc];
@@ -289,6 +299,7 @@ __device__ __forceinline__ void flush_candidates(const FaceStage* st, const Stag
 
 // Pre-test the box of staged face `slot` lane-parallel (64 pixels per round) and append the
 // passing pixels to the candidate list; flushes first whenever a round could overflow it.
+template <int G>
 __device__ __forceinline__ void collect_face(const EdgeTest& et_in, int slot, int x0, int y0, int bw, int bh,
                                              FaceStage* st, const StageOwner& own, unsigned* cand, int& count,
                                              const Camera* __restrict__ cams, bool one_view, int bc0,
@@ -298,7 +309,7 @@ __device__ __forceinline__ void collect_face(const EdgeTest& et_in, int slot, in
   for (int base = 0; base < area; base += 64) {
     if (count > kCandCap - 64) {
       __syncthreads();
-      flush_candidates(st, own, cand, count, cams, one_view, bc0, keys, W, H, false);
+      flush_candidates<G>(st, own, cand, count, cams, one_view, bc0, keys, W, H, false);
       __syncthreads();
       count = 0;
     }
@@ -331,17 +342,35 @@ __device__ __forceinline__ EdgeTest readlane_edges(const EdgeTest& e, int j) {
   return r;
 }
 
-// Boxes up to this many pixels are walked by their own lane (all lanes at once, pixel by
-// pixel along the box rows); larger staged boxes are walked by the whole wavefront, one face
-// at a time.  Per-lane walks share each iteration among all the wavefront's small faces, while
-// the wavefront walk pays a per-face setup: at 100k triangles over 8 x 1024^2 views (most
-// boxes 17-128 px) 64 was the fastest of 16, 32, 64, 96, 128 and 256.
-constexpr int kTinyBox = 64;
+// Boxes up to this many pixels are walked line by line by their own lanes, all faces of the
+// wavefront at once (BoxLines); larger staged boxes, which only a raised large-face threshold
+// brings here, are walked by the whole wavefront, one face at a time.
+constexpr int kLineBox = 256;
 
-// One wavefront per 64 consecutive (b, c, face) items (wg: the mesh's own logical block).
-// Faces with bounding boxes up to large_box pixels are staged and rasterised here (pre-test,
-// compaction, exact test); larger ones are appended to `large` for k_raster_large.
+// Inclusive sum over the 64 lanes (DPP: shifts within the rows of 16, then row broadcasts).
+__device__ __forceinline__ int wave_inclusive_sum(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);   // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);   // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);   // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1, 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2, 3
+  return x;
+}
+
+// One wavefront per 64 / G consecutive (b, c, face) items, G lanes to a face (wg: the mesh's own
+// logical block).  Faces with bounding boxes up to large_box pixels are staged and rasterised
+// here (line spans, compaction, exact test); larger ones are appended to `large` for
+// k_raster_large.
+// The G lanes of a face take its lines in turn.  On every step each lane finds the span of its
+// line, a wave sum of the span lengths gives each lane its place in the candidate list, and the
+// lanes write their spans there; a full list (always a multiple of 64) is tested and emptied.
+// Bound by VALU issue.  The spans replace an edge test of every box pixel, one pixel of 64 boxes
+// per step with 13.75 of the 64 lanes passing on average at 100k triangles over 8 x 1024^2 views:
+// 0.249 -> 0.153 ms there, 0.434 -> 0.330 ms at 200k triangles over 16 x 1024^2.
+template <int G>
 __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
+  constexpr int kFaces = 64 / G;
   const TriSetup* __restrict__ tris = ra.tris;
   const int32_t* __restrict__ faces = ra.faces;
   const float4* __restrict__ proj = ra.proj;
@@ -350,16 +379,17 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
   unsigned int* __restrict__ large_count = ra.large_count;
   int4* __restrict__ large = ra.large;
   const int B = ra.B, C = ra.C, N = ra.N, F = ra.F, W = ra.W, H = ra.H, large_box = ra.large_box, mesh_id = ra.mesh_id;
-  __shared__ FaceStage st[64];
+  __shared__ FaceStage st[kFaces];
   __shared__ unsigned cand[kCandCap];
-  const int lane = threadIdx.x;
-  const int64_t i = wg * 64 + lane;
+  const int lane = threadIdx.x, slot = lane / G, sub = lane % G;
+  const int64_t i = wg * kFaces + slot;
   const bool in_range = i < (int64_t)B * C * F;
   const int f = in_range ? (int)(i % F) : 0;
   const int bc = in_range ? (int)(i / F) : 0;
   bool small = false, to_queue = false;
   EdgeTest et;
   et.on = false;
+  for (int k = 0; k < 3; ++k) et.a[k] = et.b[k] = et.c[k] = 0.f;
   int bw = 0, bh = 0, fx0 = 0, fy0 = 0;
   if (in_range) {
     const RasterFace r = load_face(faces, proj + (size_t)bc * N, f, W, H);
@@ -367,10 +397,10 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
       bw = r.bx.x1 - r.bx.x0 + 1;
       bh = r.bx.y1 - r.bx.y0 + 1;
       if ((int64_t)bw * bh > large_box) {
-        to_queue = true;
+        to_queue = sub == 0;
       } else {
         small = true;
-        stage_face(&st[lane], tris[(size_t)(bc / C) * F + f], r.p0.z, r.p1.z, r.p2.z);
+        if (sub == 0) stage_face(&st[slot], tris[(size_t)(bc / C) * F + f], r.p0.z, r.p1.z, r.p2.z);
         et = edge_test(r.p0, r.p1, r.p2);
         fx0 = r.bx.x0;
         fy0 = r.bx.y0;
@@ -396,45 +426,51 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
   const StageOwner own{f, bc, fx0, fy0, bw};
   __syncthreads();
   int count = 0;
-  // tiny boxes: each lane walks its own box; pixel p of every lane's face per iteration
-  const int my_area = small && bw * bh <= kTinyBox ? bw * bh : 0;
-  int dx = 0, dy = 0;     // pixel p of this lane's box, stepped along its rows
-  EdgeWalk walk;
-  walk.start(et, fx0, fy0, bw);
-  for (int p = 0; __ballot(p < my_area); ++p) {
-    if (count > kCandCap - 64) {
+  const bool packed = cand_packed(W, H);
+  const bool by_line = small && bw * bh <= kLineBox;
+  BoxLines bl;
+  bl.start(et, fx0, fy0, bw, bh);
+  const int lines = by_line ? bl.lines : 0;
+  const unsigned step = cand_word(packed, false, 0, bl.columns ? 0 : 1, bl.columns ? 1 : 0, bl.columns ? 0 : 1,
+                                  bl.columns ? 1 : 0, bw);
+  for (int ln = sub; __ballot(ln < lines); ln += G) {
+    int first = 0;
+    int rem = ln < lines ? bl.span(ln, first) : 0;
+    const int incl = wave_inclusive_sum(rem);
+    int total = __builtin_amdgcn_readlane(incl, 63);
+    int pos = count + incl - rem;
+    const int dx = bl.columns ? ln : first, dy = bl.columns ? first : ln;
+    unsigned word = cand_word(packed, false, slot, fx0 + dx, fy0 + dy, dx, dy, bw);
+    for (;;) {
+      for (; rem > 0 && pos < kCandCap; --rem, ++pos, word += step) cand[pos] = word;
+      if (count + total <= kCandCap) break;
       __syncthreads();
-      flush_candidates(st, own, cand, count, cams, one_view, bc0, keys, W, H, false);
+      flush_candidates<G>(st, own, cand, kCandCap, cams, one_view, bc0, keys, W, H, false);
       __syncthreads();
+      total -= kCandCap - count;
+      pos -= kCandCap;
       count = 0;
     }
-    const bool pass = p < my_area && walk.pass(et.on);
-    const unsigned word = cand_word(cand_packed(W, H), false, lane, fx0 + dx, fy0 + dy, dx, dy, bw);
-    const bool row_end = ++dx == bw;
-    if (row_end) { dx = 0; ++dy; }
-    walk.step(et, row_end);
-    const uint64_t m = __ballot(pass);
-    if (pass) {
-      const int off = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-      cand[count + off] = word;
-    }
-    count += __popcll(m);
+    count += total;
   }
   // larger staged boxes: the whole wavefront walks one box at a time
-  uint64_t todo = __ballot(small && my_area == 0);
+  uint64_t todo = __ballot(small && !by_line && sub == 0);
   while (todo) {
     const int j = __ffsll((unsigned long long)todo) - 1;
     todo &= todo - 1;
     const EdgeTest ej = readlane_edges(et, j);
     const int x0 = __builtin_amdgcn_readlane(fx0, j), y0 = __builtin_amdgcn_readlane(fy0, j);
     const int jbw = __builtin_amdgcn_readlane(bw, j), jbh = __builtin_amdgcn_readlane(bh, j);
-    collect_face(ej, j, x0, y0, jbw, jbh, st, own, cand, count, cams, one_view, bc0, keys, W, H);
+    collect_face<G>(ej, j / G, x0, y0, jbw, jbh, st, own, cand, count, cams, one_view, bc0, keys, W, H);
   }
   __syncthreads();
-  flush_candidates(st, own, cand, count, cams, one_view, bc0, keys, W, H, false);
+  flush_candidates<G>(st, own, cand, count, cams, one_view, bc0, keys, W, H, false);
 }
 
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) k_raster(RasterArgs ra) { raster_body(ra, xcd_contiguous(blockIdx.x, gridDim.x)); }
+template <int G>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) k_raster(RasterArgs ra) {
+  raster_body<G>(ra, xcd_contiguous(blockIdx.x, gridDim.x));
+}
 
 // The depth pass's large-face test alone, so that the large-face pass can run beside the depth
 // pass: the (view, face) items whose bounding boxes exceed the threshold are appended to the
@@ -468,7 +504,7 @@ __global__ void __launch_bounds__(64) k_classify_large(RasterArgs ra) {
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) k_raster_multi(MeshTable<RasterArgs> t) {
   const MeshSlice m = t.find((unsigned)xcd_contiguous(blockIdx.x, gridDim.x));
   const RasterArgs a = t.load(m.mesh);
-  raster_body(a, m.local);
+  raster_body<1>(a, m.local);
 }
 
 // One large face (bc, f) rasterised by the whole wavefront.  Instead of the whole bounding box
@@ -510,7 +546,7 @@ __device__ __forceinline__ void raster_large_face(const TriSetup* __restrict__ t
     for (int q0 = 0; q0 < total; q0 += 64) {
       if (count > kCandCapLarge - 64) {
         __syncthreads();
-        flush_candidates(st, own, cand, count, cams, true, bc, keys, W, H, true, marks);
+        flush_candidates<1>(st, own, cand, count, cams, true, bc, keys, W, H, true, marks);
         __syncthreads();
         count = 0;
       }
@@ -537,7 +573,7 @@ __device__ __forceinline__ void raster_large_face(const TriSetup* __restrict__ t
     }
   }
   __syncthreads();
-  flush_candidates(st, own, cand, count, cams, true, bc, keys, W, H, true, marks);
+  flush_candidates<1>(st, own, cand, count, cams, true, bc, keys, W, H, true, marks);
 }
 
 // Persistent wavefronts drain the large-face queue: wavefront w rasterises faces w, w + G,
@@ -729,6 +765,16 @@ hipError_t launch_raster_large_multi(const RasterMesh* meshes, unsigned int* cou
   return hipGetLastError();
 }
 
+static void launch_raster(const ForwardPlan& p, const RasterArgs& ra, hipStream_t s) {
+  const int64_t items = (int64_t)ra.B * ra.C * ra.F;
+  if (p.raster_items <= kRasterItems16)
+    hipLaunchKernelGGL(k_raster<16>, dim3(blocks_for(items, 4)), dim3(64), 0, s, ra);
+  else if (p.raster_items <= kRasterItems4)
+    hipLaunchKernelGGL(k_raster<4>, dim3(blocks_for(items, 16)), dim3(64), 0, s, ra);
+  else
+    hipLaunchKernelGGL(k_raster<1>, dim3(blocks_for(items, 64)), dim3(64), 0, s, ra);
+}
+
 hipError_t launch_forward_raster(const ForwardPlan& p, hipStream_t s) {
   const int B = p.B, C = p.C, N = p.N, F = p.F;
   {
@@ -772,7 +818,7 @@ hipError_t launch_forward_raster(const ForwardPlan& p, hipStream_t s) {
     ra.queue_large = 0;
     {
       ProfScope ps(p.prof, "k_raster", s);
-      hipLaunchKernelGGL(k_raster, dim3(blocks_for((int64_t)B * C * F, 64)), dim3(64), 0, s, ra);
+      launch_raster(p, ra, s);
     }
     const hipError_t e_main = hipGetLastError();
     e = hipEventRecord(p.join, p.side);
@@ -786,7 +832,7 @@ hipError_t launch_forward_raster(const ForwardPlan& p, hipStream_t s) {
     if (e != hipSuccess) return e;
   } else {
     ProfScope ps(p.prof, "k_raster", s);
-    hipLaunchKernelGGL(k_raster, dim3(blocks_for((int64_t)B * C * F, 64)), dim3(64), 0, s, raster_args(p));
+    launch_raster(p, raster_args(p), s);
   }
   if (!p.shared_queue) {
     ProfScope ps(p.prof, "k_raster_large", s);

@@ -207,6 +207,8 @@ struct ForwardPlan {
   int mesh_id;                       // written into the queue entries
   bool shared_queue;                 // the queue is shared by several meshes: the caller clears
                                      // the counters and drains it (k_raster_large_multi)
+  int64_t raster_items;              // (view, face) items whose depth passes share the GPU: this
+                                     // mesh's, or those of every mesh of a multi-mesh run
   int large_box;                     // bounding boxes above this many pixels go to the queue
   // tile-binned depth pass (when tiled): per-tile face bins, their counts and the large-face
   // marks; counts and marks are zero between calls (the tile kernel resets them)

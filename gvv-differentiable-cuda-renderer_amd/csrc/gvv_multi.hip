@@ -269,6 +269,7 @@ int plan_all(Multi* m, const gvv_mesh_io* io, bool backward, hipStream_t s, std:
     fp[i].large = m->large.p;
     fp[i].mesh_id = i;
     fp[i].shared_queue = true;
+    fp[i].raster_items = (int64_t)queue;
     t[i] = raster_mesh(fp[i]);
   }
   if (m->host_table.size() != t.size() ||

@@ -13,7 +13,8 @@ namespace gvv {
 // triangles at the renderer's scale the farthest accepted pixel lay 7e-4 px outside an edge
 // (tests/edge_margin_check.hip), so 1/32 px leaves a factor of 45.  The pre-test is disabled
 // (every bounding-box pixel takes the exact test) when a vertex is near or behind the camera
-// plane, when coordinates are huge, or when the projected triangle is degenerate.
+// plane, when coordinates are huge (beyond 65536 px an edge value's own rounding, 3 ulp of the
+// coordinate, would come near the margin), or when the projected triangle is degenerate.
 constexpr float kEdgeMargin = 0.03125f;
 
 struct EdgeTest {
@@ -31,7 +32,7 @@ GVV_HD EdgeTest edge_test(float4 p0, float4 p1, float4 p2) {
   e.on = false;
   const float px[3] = {p0.x, p1.x, p2.x}, py[3] = {p0.y, p1.y, p2.y}, pz[3] = {p0.z, p1.z, p2.z};
   for (int i = 0; i < 3; ++i)
-    if (!(pz[i] >= 1.0f) || !(fabsf(px[i]) <= 1e6f) || !(fabsf(py[i]) <= 1e6f)) return e;
+    if (!(pz[i] >= 1.0f) || !(fabsf(px[i]) <= 65536.f) || !(fabsf(py[i]) <= 65536.f)) return e;
   const float area2 = (px[1] - px[0]) * (py[2] - py[0]) - (py[1] - py[0]) * (px[2] - px[0]);
   if (!(fabsf(area2) >= 1e-3f)) return e;
   const float s = area2 > 0.f ? 1.f : -1.f;
@@ -68,6 +69,61 @@ struct EdgeWalk {
   GVV_HD bool pass(bool on) const { return !on || (e[0] >= 0.f && e[1] >= 0.f && e[2] >= 0.f); }
   GVV_HD void step(const EdgeTest& t, bool row_end) {
     for (int i = 0; i < 3; ++i) e[i] += row_end ? w[i] : t.a[i];
+  }
+};
+
+// Approximate reciprocal and reciprocal square root (1 ulp on the device): only for the
+// pre-test, whose margin is thousands of times their rounding.
+GVV_HD float approx_rcp(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_rcpf(x);
+#else
+  return 1.f / x;
+#endif
+}
+
+// The pixels of a box that the pre-test keeps, line by line: lines run along the box's longer
+// side (rows, or columns of a tall box), and on each line the kept pixels are one interval,
+// because each edge bounds the position along the line from one side.  An edge's bound moves
+// linearly from line to line (t + ln * s), so a line costs three FMAs instead of three edge
+// values per pixel.
+// Rounding: with e0 the edge value at the box's first pixel and ea the edge's slope along the
+// line, a bound is -(e0 + el ln) / ea.  Its error is a few ulp of the edge value's terms (under
+// 2e-3 px for coordinates up to 65536, the limit of edge_test) divided by |ea|, while the
+// margin moves the bound outwards by kEdgeMargin / |ea|: the margin's factor over the error
+// does not depend on ea.  An edge parallel to the lines (ea = 0) bounds nothing here.
+struct BoxLines {
+  float t[3], s[3];            // bound of edge i on line ln, in pixels from the line's start
+  bool lower[3], upper[3];     // which side it bounds
+  int lines, len;              // lines of the box and pixels per line
+  bool columns;                // lines are columns (the box is taller than wide)
+  GVV_HD void start(const EdgeTest& e, int x0, int y0, int bw, int bh) {
+    columns = bh > bw;
+    lines = columns ? bw : bh;
+    len = columns ? bh : bw;
+    const float x = x0 + 0.5f, y = y0 + 0.5f;
+    for (int i = 0; i < 3; ++i) {
+      const float ea = columns ? e.b[i] : e.a[i], el = columns ? e.a[i] : e.b[i];
+      const float r = approx_rcp(ea);
+      t[i] = -(e.a[i] * x + e.b[i] * y + e.c[i]) * r;
+      s[i] = -el * r;
+      lower[i] = e.on && ea > 0.f;
+      upper[i] = e.on && ea < 0.f;
+    }
+  }
+  // first kept pixel of line ln and how many follow from it (0: none); NaN bounds (an infinite
+  // slope at line 0) bound nothing
+  GVV_HD int span(int ln, int& first) const {
+    float lo = 0.f, hi = (float)(len - 1);
+    for (int i = 0; i < 3; ++i) {
+      const float b = fmaf((float)ln, s[i], t[i]);
+      if (lower[i]) lo = fmaxf(lo, b);
+      if (upper[i]) hi = fminf(hi, b);
+    }
+    first = 0;
+    if (!(lo <= hi)) return 0;
+    first = (int)ceilf(lo);
+    return (int)floorf(hi) - first + 1;
   }
 };
 
