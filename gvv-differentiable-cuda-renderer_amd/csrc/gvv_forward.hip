@@ -179,7 +179,9 @@ __global__ void __launch_bounds__(256) k_vertices_multi(MeshTable<VertexArgs> t)
   vertices_body(a, m.local);
 }
 
-constexpr int kLargeWorkgroups = 4096;
+constexpr unsigned kLargeWaves = 8192;           // persistent wavefronts of the large-face pass
+constexpr unsigned kLargeItems = 8192;          // face parts that a short queue is split into
+constexpr int kLargePart = 512;                   // box pixels below which a large face is not split further
 // (view, face) items up to which the depth pass gives 16, or 4, lanes to a face instead of one.
 // A wavefront's time is a serial chain over its faces' lines and candidates, so with fewer than
 // about 4096 wavefronts the chain, not the chip, is the kernel's time: 20,480 items (4 x 256^2
@@ -358,6 +360,26 @@ __device__ __forceinline__ int wave_inclusive_sum(int x) {
   return x;
 }
 
+// Appends every lane's span (rem candidates: word, word + step, ...) to the wavefront's list of
+// CAP candidates, each span in one piece in lane order; a full list (a multiple of 64) is handed
+// to flush() and starts again.  total: the sum of rem over the lanes, incl its inclusive prefix.
+template <int CAP, class Flush>
+__device__ __forceinline__ void append_spans(unsigned* cand, int& count, int rem, int incl, int total, unsigned word,
+                                             unsigned step, Flush&& flush) {
+  int pos = count + incl - rem;
+  for (;;) {
+    for (; rem > 0 && pos < CAP; --rem, ++pos, word += step) cand[pos] = word;
+    if (count + total <= CAP) break;
+    wave_sync();
+    flush(CAP);
+    wave_sync();
+    total -= CAP - count;
+    pos -= CAP;
+    count = 0;
+  }
+  count += total;
+}
+
 // One wavefront per 64 / G consecutive (b, c, face) items, G lanes to a face (wg: the mesh's own
 // logical block).  Faces with bounding boxes up to large_box pixels are staged and rasterised
 // here (line spans, compaction, exact test); larger ones are appended to `large` for
@@ -409,7 +431,6 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
   }
   // large faces go to the queue with one atomic per wavefront (the cursor is a single word
   // that every wavefront of the launch would otherwise hit once per face)
-  if (!ra.queue_large) to_queue = false;
   const uint64_t qm = __ballot(to_queue);
   if (qm) {
     unsigned int base = 0;
@@ -435,23 +456,13 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
                                   bl.columns ? 1 : 0, bw);
   for (int ln = sub; __ballot(ln < lines); ln += G) {
     int first = 0;
-    int rem = ln < lines ? bl.span(ln, first) : 0;
+    const int rem = ln < lines ? bl.span(ln, first) : 0;
     const int incl = wave_inclusive_sum(rem);
-    int total = __builtin_amdgcn_readlane(incl, 63);
-    int pos = count + incl - rem;
     const int dx = bl.columns ? ln : first, dy = bl.columns ? first : ln;
-    unsigned word = cand_word(packed, false, slot, fx0 + dx, fy0 + dy, dx, dy, bw);
-    for (;;) {
-      for (; rem > 0 && pos < kCandCap; --rem, ++pos, word += step) cand[pos] = word;
-      if (count + total <= kCandCap) break;
-      __syncthreads();
-      flush_candidates<G>(st, own, cand, kCandCap, cams, one_view, bc0, keys, W, H, false);
-      __syncthreads();
-      total -= kCandCap - count;
-      pos -= kCandCap;
-      count = 0;
-    }
-    count += total;
+    const unsigned word = cand_word(packed, false, slot, fx0 + dx, fy0 + dy, dx, dy, bw);
+    append_spans<kCandCap>(cand, count, rem, incl, __builtin_amdgcn_readlane(incl, 63), word, step, [&](int n) {
+      flush_candidates<G>(st, own, cand, n, cams, one_view, bc0, keys, W, H, false);
+    });
   }
   // larger staged boxes: the whole wavefront walks one box at a time
   uint64_t todo = __ballot(small && !by_line && sub == 0);
@@ -472,115 +483,87 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) k_
   raster_body<G>(ra, xcd_contiguous(blockIdx.x, gridDim.x));
 }
 
-// The depth pass's large-face test alone, so that the large-face pass can run beside the depth
-// pass: the (view, face) items whose bounding boxes exceed the threshold are appended to the
-// queue (one atomic per wavefront), by the same box computation as k_raster, which then skips
-// them.
-__global__ void __launch_bounds__(64) k_classify_large(RasterArgs ra) {
-  const int lane = threadIdx.x;
-  const int64_t i = (int64_t)blockIdx.x * 64 + lane;
-  bool to_queue = false;
-  int f = 0, bc = 0;
-  if (i < (int64_t)ra.B * ra.C * ra.F) {
-    f = (int)(i % ra.F);
-    bc = (int)(i / ra.F);
-    const RasterFace r = load_face(ra.faces, ra.proj + (size_t)bc * ra.N, f, ra.W, ra.H);
-    if (r.bx.x0 <= r.bx.x1 && r.bx.y0 <= r.bx.y1) {
-      const int bw = r.bx.x1 - r.bx.x0 + 1, bh = r.bx.y1 - r.bx.y0 + 1;
-      to_queue = (int64_t)bw * bh > ra.large_box;
-    }
-  }
-  const uint64_t qm = __ballot(to_queue);
-  if (!qm) return;
-  unsigned int base = 0;
-  if (lane == __ffsll((unsigned long long)qm) - 1) base = atomicAdd(ra.large_count, (unsigned)__popcll(qm));
-  base = __builtin_amdgcn_readlane(base, __ffsll((unsigned long long)qm) - 1);
-  if (to_queue) {
-    const unsigned off = __builtin_amdgcn_mbcnt_hi((unsigned)(qm >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)qm, 0u));
-    ra.large[base + off] = make_int4(bc, f, ra.mesh_id, 0);
-  }
-}
-
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) k_raster_multi(MeshTable<RasterArgs> t) {
   const MeshSlice m = t.find((unsigned)xcd_contiguous(blockIdx.x, gridDim.x));
   const RasterArgs a = t.load(m.mesh);
   raster_body<1>(a, m.local);
 }
 
-// One large face (bc, f) rasterised by the whole wavefront.  Instead of the whole bounding box
-// the wavefront walks, 64 rows at a time, the conservative span of each row (row_span; a wave
-// prefix sum turns spans into pixel indices), applies the edge pre-test, compacts and runs the
-// exact test as k_raster does.
+// Part `part` of `parts` of one large face (bc, f), rasterised by the whole wavefront: lines part,
+// part + parts, ... of its box.  The spans of 64 lines are found at once, one per lane
+// (BoxLines).  They go to the candidate list one span at a time, 64 pixels per step, or, where
+// they are shorter than they are many (a sliver across its box), all at once, one pixel of each
+// per step.  Full lists take the exact test as in k_raster.
 __device__ __forceinline__ void raster_large_face(const TriSetup* __restrict__ tris, const int32_t* __restrict__ faces,
                                                   const float4* __restrict__ proj, const Camera* __restrict__ cams,
                                                   unsigned long long* __restrict__ keys, int C, int N, int F, int W,
-                                                  int H, int bc, int f, FaceStage* st, unsigned* cand, int* s_xl,
-                                                  int* s_start, TileMarks marks) {
+                                                  int H, int bc, int f, int part, int parts, FaceStage* st,
+                                                  unsigned* cand, TileMarks marks) {
   const RasterFace r = load_face(faces, proj + (size_t)bc * N, f, W, H);
   const int bw = r.bx.x1 - r.bx.x0 + 1, bh = r.bx.y1 - r.bx.y0 + 1;
-  __syncthreads();
-  if (threadIdx.x == 0) stage_face(&st[0], tris[(size_t)(bc / C) * F + f], r.p0.z, r.p1.z, r.p2.z);
+  parts = max(1, min(parts, min(min(bw, bh), (int)(((int64_t)bw * bh) / kLargePart))));
+  if (part >= parts) return;
+  BoxLines bl;
+  bl.start(edge_test(r.p0, r.p1, r.p2), r.bx.x0, r.bx.y0, bw, bh);
+  const int lane = threadIdx.x & 63;
+  wave_sync();
+  if (lane == 0) stage_face(&st[0], tris[(size_t)(bc / C) * F + f], r.p0.z, r.p1.z, r.p2.z);
   const StageOwner own{f, bc, r.bx.x0, r.bx.y0, bw};
-  const EdgeTest et = edge_test(r.p0, r.p1, r.p2);
-  __syncthreads();
+  wave_sync();
+  const bool packed = cand_packed(W, H);
+  const unsigned step = cand_word(packed, true, 0, bl.columns ? 0 : 1, bl.columns ? 1 : 0, bl.columns ? 0 : 1,
+                                  bl.columns ? 1 : 0, bw);
   int count = 0;
-  const int lane = threadIdx.x;
-  for (int rbase = 0; rbase < bh; rbase += 64) {
-    // this lane's row: span and length; inclusive scan of the lengths over the wave
-    const int y = r.bx.y0 + rbase + lane;
-    int xl = 0, xr = -1;
-    if (rbase + lane < bh) row_span(et, y, r.bx.x0, r.bx.x1, xl, xr);
-    const int len = xr >= xl ? xr - xl + 1 : 0;
-    int incl = len;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int t = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += t;
+  const auto flush = [&](int n) {
+    flush_candidates<1>(st, own, cand, n, cams, true, bc, keys, W, H, true, marks);
+  };
+  for (int l0 = part; l0 < bl.lines; l0 += 64 * parts) {
+    const int ln = l0 + lane * parts;
+    int first = 0;
+    const int len = ln < bl.lines ? bl.span(ln, first) : 0;
+    const int dx = bl.columns ? ln : first, dy = bl.columns ? first : ln;
+    const unsigned word = cand_word(packed, true, 0, r.bx.x0 + dx, r.bx.y0 + dy, dx, dy, bw);
+    uint64_t todo = __ballot(len > 0);
+    const int incl = wave_inclusive_sum(len), total = __builtin_amdgcn_readlane(incl, 63), spans = __popcll(todo);
+    if (2 * total <= spans * spans) {
+      append_spans<kCandCapLarge>(cand, count, len, incl, total, word, step, flush);
+      continue;
     }
-    const int total = __shfl(incl, 63, 64);
-    if (total == 0) continue;
-    __syncthreads();
-    s_xl[lane] = xl;
-    s_start[lane] = incl - len;
-    __syncthreads();
-    for (int q0 = 0; q0 < total; q0 += 64) {
-      if (count > kCandCapLarge - 64) {
-        __syncthreads();
-        flush_candidates<1>(st, own, cand, count, cams, true, bc, keys, W, H, true, marks);
-        __syncthreads();
-        count = 0;
+    for (; todo; todo &= todo - 1) {
+      const int j = __ffsll((unsigned long long)todo) - 1;
+      const unsigned word_j = __builtin_amdgcn_readlane(word, j);
+      const int len_j = __builtin_amdgcn_readlane(len, j);
+      for (int k0 = 0; k0 < len_j; k0 += 64) {
+        if (count > kCandCapLarge - 64) {
+          wave_sync();
+          flush(count);
+          wave_sync();
+          count = 0;
+        }
+        if (k0 + lane < len_j) cand[count + lane] = word_j + (unsigned)(k0 + lane) * step;
+        count += min(64, len_j - k0);
       }
-      const int q = q0 + lane;
-      bool pass = false;
-      int p = 0;
-      if (q < total) {
-        // the row holding span pixel q: the last row whose start is <= q
-        int row = 0;
-#pragma unroll
-        for (int step = 32; step > 0; step >>= 1)
-          if (row + step < 64 && s_start[row + step] <= q) row += step;
-        const int x = s_xl[row] + (q - s_start[row]);
-        const int yy = r.bx.y0 + rbase + row;
-        pass = et.pass(x + 0.5f, yy + 0.5f);
-        p = (int)cand_word(cand_packed(W, H), true, 0, x, yy, x - r.bx.x0, yy - r.bx.y0, bw);
-      }
-      const uint64_t m = __ballot(pass);
-      if (pass) {
-        const int off = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-        cand[count + off] = (unsigned)p;
-      }
-      count += __popcll(m);
     }
   }
-  __syncthreads();
-  flush_candidates<1>(st, own, cand, count, cams, true, bc, keys, W, H, true, marks);
+  wave_sync();
+  flush(count);
 }
 
-// Persistent wavefronts drain the large-face queue: wavefront w rasterises faces w, w + G,
-// w + 2G, ... (G wavefronts) up to the queue length written by k_raster (raster_large_face).
-// A shared atomic cursor would balance better, but every wavefront taking every item from one
-// word serialises on that word's memory-side atomics: 4k cursor atomics took longer than the
-// faces themselves.
+// Persistent wavefronts drain the large-face queue, whose length k_raster wrote: n faces are split
+// into kLargeItems / n parts each (at least one; a face of few pixels is split less), and of G
+// wavefronts, w takes parts w, w + G, ...  A shared atomic cursor would balance better, but every
+// wavefront taking every item from one word serialises on that word's memory-side atomics: 4k
+// cursor atomics took longer than the faces themselves.
+// A part repeats the face's setup (about 300 instructions) but no pixel's work, so that a short
+// queue fills the chip: 1,280 faces of about 3,000 px each took 373 us with one wavefront per
+// face.  The pass follows k_raster on the same stream: beside it, on a second stream with a
+// kernel of its own to fill the queue, the fork and join left 6 and 10 us of idle time per
+// forward, as much as the overlap saved (100k faces over 8 x 1024^2: 651 us forward + backward
+// beside, 662 in line; 304 against 278 for the 1,280 faces, 173 against 161 for 6 x 333 x 477).
+__device__ __forceinline__ int large_parts(unsigned n_large) {
+  return (int)min(max(kLargeItems / max(n_large, 1u), 1u), 64u);
+}
+
 __global__ void __launch_bounds__(64) k_raster_large(const TriSetup* __restrict__ tris, const int32_t* __restrict__ faces,
                                                      const float4* __restrict__ proj, const Camera* __restrict__ cams,
                                                      unsigned long long* __restrict__ keys,
@@ -588,11 +571,13 @@ __global__ void __launch_bounds__(64) k_raster_large(const TriSetup* __restrict_
                                                      int C, int N, int F, int W, int H, TileMarks marks) {
   __shared__ FaceStage st[1];
   __shared__ unsigned cand[kCandCapLarge];
-  __shared__ int s_xl[64], s_start[64];
   const unsigned int n_large = counters[0];
-  for (unsigned int item = blockIdx.x; item < n_large; item += gridDim.x)
-    raster_large_face(tris, faces, proj, cams, keys, C, N, F, W, H, large[item].x, large[item].y, st, cand, s_xl,
-                      s_start, marks);
+  const unsigned int parts = (unsigned)large_parts(n_large);
+  for (unsigned int item = blockIdx.x; item < n_large * parts; item += gridDim.x) {
+    const int4 e = large[item / parts];
+    raster_large_face(tris, faces, proj, cams, keys, C, N, F, W, H, e.x, e.y, (int)(item % parts), (int)parts, st, cand,
+                      marks);
+  }
 }
 
 // The same over a queue shared by several meshes: each entry names its mesh, whose raster
@@ -602,13 +587,13 @@ __global__ void __launch_bounds__(64) k_raster_large_multi(const RasterMesh* __r
                                                            const int4* __restrict__ large) {
   __shared__ FaceStage st[1];
   __shared__ unsigned cand[kCandCapLarge];
-  __shared__ int s_xl[64], s_start[64];
   const unsigned int n_large = counters[0];
-  for (unsigned int item = blockIdx.x; item < n_large; item += gridDim.x) {
-    const int4 e = large[item];
+  const unsigned int parts = (unsigned)large_parts(n_large);
+  for (unsigned int item = blockIdx.x; item < n_large * parts; item += gridDim.x) {
+    const int4 e = large[item / parts];
     const RasterMesh m = meshes[e.z];
-    raster_large_face(m.tris, m.faces, m.proj, m.cams, m.keys, m.C, m.N, m.F, m.W, m.H, e.x, e.y, st, cand, s_xl,
-                      s_start, m.marks);
+    raster_large_face(m.tris, m.faces, m.proj, m.cams, m.keys, m.C, m.N, m.F, m.W, m.H, e.x, e.y, (int)(item % parts),
+                      (int)parts, st, cand, m.marks);
   }
 }
 
@@ -742,7 +727,6 @@ RasterArgs raster_args(const ForwardPlan& p) {
   a.large_count = p.counters; a.large = p.large;
   a.B = p.B; a.C = p.C; a.N = p.N; a.F = p.F; a.W = p.r.W; a.H = p.r.H;
   a.large_box = p.large_box; a.mesh_id = p.mesh_id;
-  a.queue_large = 1;
   return a;
 }
 
@@ -761,7 +745,7 @@ hipError_t launch_clear_counters(unsigned int* counters, hipStream_t s) {
 
 hipError_t launch_raster_large_multi(const RasterMesh* meshes, unsigned int* counters, const int4* large,
                                      hipStream_t s) {
-  hipLaunchKernelGGL(k_raster_large_multi, dim3(kLargeWorkgroups), dim3(64), 0, s, meshes, counters, large);
+  hipLaunchKernelGGL(k_raster_large_multi, dim3(kLargeWaves), dim3(64), 0, s, meshes, counters, large);
   return hipGetLastError();
 }
 
@@ -794,38 +778,6 @@ hipError_t launch_forward_raster(const ForwardPlan& p, hipStream_t s) {
                        p.vnormal_out, p.normal_map_out, B, C, N, T);
     return hipGetLastError();
   }
-  // the large faces classified and rasterised on the handle's second stream, beside the depth
-  // pass (both take the 64-bit minimum of the same keys, so the order is free); in line when
-  // the caller's stream is being captured into a graph
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (p.side && hipStreamIsCapturing(s, &capture) != hipSuccess) capture = hipStreamCaptureStatusActive;
-  if (!p.tiled && !p.shared_queue && p.side && capture == hipStreamCaptureStatusNone) {
-    hipError_t e = hipEventRecord(p.fork, s);
-    if (e == hipSuccess) e = hipStreamWaitEvent(p.side, p.fork, 0);
-    if (e != hipSuccess) return e;
-    // from here on the second stream is joined back whatever fails in between
-    RasterArgs ra = raster_args(p);
-    {
-      ProfScope ps(p.prof, "k_classify_large", p.side);
-      hipLaunchKernelGGL(k_classify_large, dim3(blocks_for((int64_t)B * C * F, 64)), dim3(64), 0, p.side, ra);
-    }
-    {
-      ProfScope ps(p.prof, "k_raster_large", p.side);
-      hipLaunchKernelGGL(k_raster_large, dim3(kLargeWorkgroups), dim3(64), 0, p.side, p.tris, p.faces, p.proj, p.cams,
-                         p.r.keys, p.counters, p.large, C, N, F, p.r.W, p.r.H, TileMarks{});
-    }
-    const hipError_t e_side = hipGetLastError();
-    ra.queue_large = 0;
-    {
-      ProfScope ps(p.prof, "k_raster", s);
-      launch_raster(p, ra, s);
-    }
-    const hipError_t e_main = hipGetLastError();
-    e = hipEventRecord(p.join, p.side);
-    if (e == hipSuccess) e = hipStreamWaitEvent(s, p.join, 0);
-    if (e != hipSuccess) return e;
-    return e_side != hipSuccess ? e_side : e_main;
-  }
   if (p.tiled) {
     ProfScope ps(p.prof, "k_bin", s);
     hipError_t e = launch_bin(p, s);
@@ -836,7 +788,7 @@ hipError_t launch_forward_raster(const ForwardPlan& p, hipStream_t s) {
   }
   if (!p.shared_queue) {
     ProfScope ps(p.prof, "k_raster_large", s);
-    hipLaunchKernelGGL(k_raster_large, dim3(kLargeWorkgroups), dim3(64), 0, s, p.tris, p.faces, p.proj, p.cams,
+    hipLaunchKernelGGL(k_raster_large, dim3(kLargeWaves), dim3(64), 0, s, p.tris, p.faces, p.proj, p.cams,
                        p.r.keys, p.counters, p.large, C, N, F, p.r.W, p.r.H, p.tiled ? p.marks : TileMarks{});
   }
   return hipGetLastError();

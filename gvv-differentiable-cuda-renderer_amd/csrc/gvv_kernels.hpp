@@ -72,6 +72,13 @@ __device__ __forceinline__ int64_t xcd_contiguous(int64_t wg, int64_t n) {
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + j;
 }
 
+// Orders a wavefront's LDS accesses around it, for LDS that only this wavefront uses.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // One launch over several meshes: mesh i owns the blocks [start[i], start[i+1]) of the grid
 // (in the logical order, after any XCD remapping) and takes args[i].  find() is a binary search
 // over the uniform prefix table.
@@ -163,8 +170,6 @@ struct RasterArgs {
   unsigned int* large_count;         // queue length
   int4* large;                       // large-face queue
   int B, C, N, F, W, H, large_box, mesh_id;
-  int queue_large;                   // 1: append large faces to the queue; 0: skip them (queued
-                                     // already by k_classify_large)
 };
 
 struct ResolveArgs {
@@ -218,10 +223,6 @@ struct ForwardPlan {
   TileMarks marks;
   ResolveArgs r;
   Profiler* prof;
-  // the large-face pass beside the depth pass: a second stream of the handle and the events
-  // that fork it from the caller's stream after k_vertices and join it back (null: in line)
-  hipStream_t side;
-  hipEvent_t fork, join;
 };
 
 struct BackwardArgs {

@@ -34,12 +34,6 @@ struct TileFace {
 
 constexpr int kTileCand = 512;         // candidate list of one wavefront (32-bit words)
 
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Whether any pixel centre of tile (tx, ty) can pass the edge pre-test: for each edge, the
 // largest value of its (pixel-normalised) edge function over the tile's pixel-centre
 // rectangle, less a 1/64 px allowance for the rounding of this bound.

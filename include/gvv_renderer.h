@@ -65,10 +65,7 @@ void gvv_destroy(void* handle);
  * The op's target_image_out output is the target input itself (an alias); it is not handled
  * here.  Visibility ties between faces at the same integer depth resolve to the lowest face
  * id (the reference resolves them by an unsynchronised last write).
- * Work is ordered on the caller's stream.  Outside stream capture, the large-face part of the
- * depth pass runs on a second stream the handle owns, forked from and joined back to the
- * caller's stream with events inside the call, so the call's results are complete in the
- * caller's stream order as usual; under capture everything stays on the caller's stream. */
+ * Work is ordered on the caller's stream. */
 int gvv_forward(void* handle, int32_t B, int32_t texH, int32_t texW, const float* vpos, const float* vcol,
                 const float* tex, const float* sh, const float* extr, const float* intr, float* bary,
                 int32_t* face, float* render, float* vnormal, float* normal_map, void* hip_stream);

@@ -1,6 +1,6 @@
 // The line spans of the depth pass (gvv_raster.hpp BoxLines) against the exact ray/triangle
 // test: random triangles (a third slivers, some with a vertex far outside the image) seen by a
-// pinhole camera, boxes clipped to the image and up to 4096 px.  Counts the pixels that the
+// pinhole camera, boxes clipped to the image, up to 4096 px and a few of any size.  Counts the pixels that the
 // exact test accepts and the spans leave out (missed), and the least distance in px by which an
 // accepted pixel lies inside an edge's bound (slack; the pre-test's margin is 1/32 px).
 // Host only.
@@ -26,7 +26,8 @@ int main(int argc, char** argv) {
     Camera cam;
     camera_setup(E, K, cam);
     const double px_mm = dist / (1.2 * W);
-    const double size = px_mm * std::pow(10.0, -0.5 + 2.2 * U(rng));      // 0.3 .. 50 px
+    const bool big = t % 997 == 0;
+    const double size = px_mm * std::pow(10.0, -0.5 + 2.2 * U(rng)) * (big ? 30 : 1);      // 0.3 .. 50 px
     const double cx = (U(rng) - 0.5) * W * px_mm, cy = (U(rng) - 0.5) * H * px_mm, cz = G(rng) * 50;
     V3 v[3];
     float4 p[3];
@@ -42,7 +43,7 @@ int main(int argc, char** argv) {
     const Box bx = face_box(v3(p[0].x, p[0].y, p[0].z), v3(p[1].x, p[1].y, p[1].z), v3(p[2].x, p[2].y, p[2].z), W, H);
     if (bx.x0 > bx.x1 || bx.y0 > bx.y1) continue;
     const int bw = bx.x1 - bx.x0 + 1, bh = bx.y1 - bx.y0 + 1;
-    if ((long long)bw * bh > 4096) continue;
+    if ((long long)bw * bh > 4096 && !big) continue;
     ++boxes;
     area += bw * bh;
     const EdgeTest et = edge_test(p[0], p[1], p[2]);
