@@ -7,26 +7,37 @@
 //
 //   forward        O[q][p] = sum_k P[p][k] Q[q][k]   p = output channel, q = output pixel,
 //                                                    k = (kh, kw, ci)
-//   backward data  p = input channel, q = input pixel, k = (kh, kw, co); taps whose output
-//                  pixel is off the stride grid contribute zero
-//   backward wt    p = (kh, kw, ci), q = output channel, k = output pixel (split over the grid
-//                  z dimension into FP32 partials, summed by k_split_sum)
+//   backward data  p = input channel, q = input pixel, k = (kh, kw, co).  Input pixels are taken
+//                  by their residue modulo the stride: pixels of one residue class see the same
+//                  taps, so only taps on the stride grid are loaded and multiplied
+//   backward wt    p = (kh, kw, ci), q = output channel, k = output pixel
 //
 // Activations are NHWC bf16 with the channel count a multiple of 8, so that 8 consecutive k
-// are 8 consecutive channels of one tap: one 16-byte load per MFMA operand chunk.  For the
-// weight gradient the reduction runs over pixels, which are strided in NHWC; each lane then
-// gathers 8 pixels of one channel with 2-byte loads that are contiguous across the wave.
+// are 8 consecutive channels of one tap: one 16-byte load per MFMA operand chunk.
+//
+// What bounds these layers is latency: at 16 images of 256^2 the whole network is 7 GFLOP and
+// 50 MB forward (6 and 10 us at this card's rates), over layers of 3 to 128 MFMA depths with
+// 128 to 4096 output tiles of 64 x 64.  So the loads of one output tile's reduction are shared out
+// over the waves of a workgroup: each wave loads the operands of its stretch of k straight from
+// global memory into MFMA registers, all at once, with no LDS staging.  Forward and backward data
+// keep one accumulation chain per output, in k order, whatever the tile and the number of waves
+// (their results feed bf16 roundings, which another order of addition would move): the
+// accumulators go from wave to wave through LDS, and each wave adds its stretch when they arrive.
+// The chain is short next to the loads it no longer waits for (a step of 32 k is 16 cycles of a
+// dependent MFMA).  The weight gradient, an FP32 result, adds the waves' own sums at the end.
+// Staging both operands in LDS with two barriers per 32 k took 236 us for the seven forward
+// layers of 16 images and 212 us for one, 290 for backward data and 385 for the weights of 16.
 //
 // MFMA lane layout (16x16x32, wave64): lane l supplies row l%16 of A and column l%16 of B with
 // k = 8*(l/16) .. 8*(l/16)+7; it receives D[4*(l/16)+r][l%16] in accumulator r.  A is the P
-// side, B the Q side, so each lane ends with 4 consecutive p of one q: one 8-byte (bf16) or
-// 16-byte (fp32) store.
+// side, B the Q side, so each lane ends with 4 consecutive p of one q.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <string>
 
 #include "../../include/gvv_proposal.h"
+#include "gvv_kernels.hpp"
 
 namespace gvv {
 int set_last_error(const std::string& m);
@@ -36,12 +47,6 @@ namespace {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
-
-constexpr int kBK = 32;           // k per main-loop step (one MFMA depth)
-constexpr int kRow = kBK + 8;     // LDS row stride in bf16 (80 bytes: spreads rows over banks)
-constexpr int kThreads = 256;     // 4 waves, 2 x 2 over the (P, Q) tile
-
-enum Mode { kFwd = 0, kBwdData = 1, kBwdWeight = 2 };
 
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float(uint32_t(h) << 16); }
 
@@ -58,155 +63,124 @@ struct ConvGeom {
   int B, H, W, Cin, OH, OW, Cout, KS, S, PAD;
 };
 
-struct ConvArgs {
-  ConvGeom g;
-  const uint16_t* x;       // [B][H][W][Cin]       forward input (bf16)
-  const uint16_t* w;       // [Cout][KS][KS][Cin]  weights (bf16)
-  const uint16_t* wt;      // [Cin][KS][KS][Cout]  transposed weights (bf16)
-  const uint16_t* dz;      // [B][OH][OW][Cout]    gradient at the pre-activation output (bf16)
-  const float* bias;       // [Cout]
-  void* out;               // fwd: y (bf16 or f32); bwd data: dx (bf16); bwd wt: partials (f32)
-  int out_f32, relu;
-  const uint16_t* mask;    // bwd data: dx *= (mask > 0) where mask is the layer's forward input
-  int64_t k_per_split;     // bwd wt: pixels per grid-z slice (multiple of kBK)
+struct alignas(16) Words4 { uint32_t w[4]; };
+
+__device__ __forceinline__ bf16x8 as_bf16x8(const Words4& v) {
+  bf16x8 r;
+  __builtin_memcpy(&r, &v, 16);
+  return r;
+}
+
+// a / b for 0 <= a, b > 0 with a quotient that fits an int: a 32-bit division wherever it can be
+__device__ __forceinline__ int quotient(int64_t a, int b) {
+  return (a >> 32) == 0 ? int(uint32_t(a) / uint32_t(b)) : int(a / b);
+}
+
+__device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// ---- forward and backward data -----------------------------------------------------------
+// One residue class of backward data (forward: the only one): output pixels y = S yc + ry,
+// x = S xc + rx; taps kh = kh0 + kstep t, t < nty (kw likewise), reading source row
+// (y0 + dir t) with y0 = yc ymul + yadd.
+struct Taps {
+  int n;                // taps of this axis
+  int k0;               // first tap
+  int add;              // source position of pixel 0 under the first tap
+  int pixels;           // output pixels of this class along the axis
 };
 
-// GEMM extents of each mode
-__host__ __device__ inline void gemm_dims(int mode, const ConvGeom& g, int64_t& P, int64_t& Q, int64_t& K) {
-  const int64_t taps = int64_t(g.KS) * g.KS;
-  if (mode == kFwd) { P = g.Cout; Q = int64_t(g.B) * g.OH * g.OW; K = taps * g.Cin; }
-  else if (mode == kBwdData) { P = g.Cin; Q = int64_t(g.B) * g.H * g.W; K = taps * g.Cout; }
-  else { P = taps * g.Cin; Q = g.Cout; K = int64_t(g.B) * g.OH * g.OW; }
+__host__ __device__ inline Taps axis_taps(bool fwd, int KS, int S, int PAD, int in, int out, int r) {
+  Taps t;
+  if (fwd) {
+    t.n = KS; t.k0 = 0; t.add = -PAD; t.pixels = out;
+  } else {
+    t.k0 = (r + PAD) % S;
+    t.n = t.k0 < KS ? (KS - t.k0 + S - 1) / S : 0;
+    t.add = (r + PAD - t.k0) / S;
+    t.pixels = r < in ? (in - r + S - 1) / S : 0;
+  }
+  return t;
 }
 
-__device__ __forceinline__ uint4 ld16(const uint16_t* p) { return *reinterpret_cast<const uint4*>(p); }
+struct ConvArgs {
+  ConvGeom g;
+  const uint16_t* src;     // forward: x [B][H][W][Cin]; backward data: dz [B][OH][OW][Cout]
+  const uint16_t* w;       // forward: w [Cout][KS][KS][Cin]; backward data: wt [Cin][KS][KS][Cout]
+  const float* bias;       // forward: [Cout]
+  const uint16_t* mask;    // backward data: dx *= (mask > 0) where mask is the layer's forward input
+  void* out;               // forward: y (bf16 or f32); backward data: dx (bf16)
+  int out_f32, relu;
+  int wide;                // out and mask are 16-byte aligned
+  int ptiles, qtiles;      // tiles of one class
+  int classes_x;
+};
 
-// Output-pixel index -> input element offset of tap (kh, kw), channel ci; -1 off the image.
-__device__ __forceinline__ int64_t in_offset(const ConvGeom& g, int64_t pix, int kh, int kw, int ci) {
-  const int ohw = g.OH * g.OW;
-  const int img = int(pix / ohw);
-  const int r = int(pix - int64_t(img) * ohw);
-  const int oh = r / g.OW, ow = r - oh * g.OW;
-  const int ih = oh * g.S - g.PAD + kh, iw = ow * g.S - g.PAD + kw;
-  if (ih < 0 || ih >= g.H || iw < 0 || iw >= g.W) return -1;
-  return ((int64_t(img) * g.H + ih) * g.W + iw) * g.Cin + ci;
-}
-
-template <int MODE, int BP, int BQ>
-__global__ __launch_bounds__(kThreads) void k_conv(ConvArgs a) {
-  static_assert(BP % 32 == 0 && BQ % 32 == 0, "tile must split over 2 x 2 waves of 16 x 16 MFMAs");
-  constexpr int TP = BP / 32, TQ = BQ / 32;                 // MFMA tiles per wave
-  constexpr int NP = (BP * 4 + kThreads - 1) / kThreads;    // P chunks per thread per step
-  constexpr int NQ = (BQ * 4 + kThreads - 1) / kThreads;
-  __shared__ __attribute__((aligned(16))) uint16_t sP[BP * kRow];
-  __shared__ __attribute__((aligned(16))) uint16_t sQ[BQ * kRow];
-
+// 16 TP x 16 TQ outputs per workgroup of NW waves.  The k steps (of 32) are taken in stretches of up
+// to NS, wave 0 first; every wave has its next stretch's operands in flight while the accumulators
+// travel.
+// Few MFMAs go with each operand here, so the integer work around them counts: an output pixel is
+// decoded once per row of a tile, and every address is a per-lane pointer plus an offset of the
+// step.  ALIGNED (C a multiple of 32): a step lies in one tap, so that offset is uniform and is
+// kept in scalar registers; otherwise (the first layer, 8 channels) each 8-channel chunk of a lane
+// finds its own tap.
+template <bool FWD, bool ALIGNED, int TP, int TQ, int NW, int NS>
+__global__ __launch_bounds__(64 * NW) void k_conv(ConvArgs a) {
+  constexpr int BP = 16 * TP, BQ = 16 * TQ;
+  constexpr int kRow = BP + 4;                          // LDS row of one q, padded
+  __shared__ __attribute__((aligned(16))) float tile[BQ * kRow];   // the accumulators between waves, [q][p]
+  __shared__ int64_t s_out[BQ];                         // output offset of each q; -1 past the end
   const ConvGeom g = a.g;
-  int64_t P, Q, K;
-  gemm_dims(MODE, g, P, Q, K);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t q0 = int64_t(blockIdx.x) * BQ;
-  const int64_t p0 = int64_t(blockIdx.y) * BP;
-  int64_t kbeg = 0, kend = K;
-  if (MODE == kBwdWeight) {
-    kbeg = int64_t(blockIdx.z) * a.k_per_split;
-    kend = kbeg + a.k_per_split < K ? kbeg + a.k_per_split : K;
-  }
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const unsigned id = (unsigned)gvv::xcd_contiguous(blockIdx.x, gridDim.x);
+  const unsigned per_class = (unsigned)a.ptiles * (unsigned)a.qtiles;
+  const int cls = (int)(id / per_class);
+  const unsigned rest = id - (unsigned)cls * per_class;
+  const int qt = (int)(rest / (unsigned)a.ptiles), pt = (int)(rest - (unsigned)qt * (unsigned)a.ptiles);
+  const int ry = FWD ? 0 : cls / a.classes_x, rx = FWD ? 0 : cls - ry * a.classes_x;
+  const Taps ty = axis_taps(FWD, g.KS, g.S, g.PAD, g.H, g.OH, ry), tx = axis_taps(FWD, g.KS, g.S, g.PAD, g.W, g.OW, rx);
+  const int C = FWD ? g.Cin : g.Cout, P = FWD ? g.Cout : g.Cin;
+  const int SH = FWD ? g.H : g.OH, SW = FWD ? g.W : g.OW;                     // source image
+  const int DH = FWD ? g.OH : g.H, DW = FWD ? g.OW : g.W;                     // output image
+  const int kstep = FWD ? 1 : g.S, dir = FWD ? 1 : -1, mul = FWD ? g.S : 1;
+  const int64_t Q = int64_t(g.B) * ty.pixels * tx.pixels;
+  const int64_t q0 = int64_t(qt) * BQ;
+  if (q0 >= Q) return;                                  // smaller classes have fewer tiles
+  const int p0 = pt * BP;
+  const unsigned C8 = (unsigned)C >> 3;
+  const unsigned chunks = (unsigned)(ty.n * tx.n) * C8;                       // 8-channel chunks of k
+  const unsigned steps = (chunks + 3) / 4;
+  const int row = lane & 15, kg = lane >> 4;
 
-  // Per-thread chunk coordinates: in forward and backward-data a chunk is (row, k-chunk) with
-  // 4 consecutive threads on one row (64 contiguous bytes); in backward-weight consecutive
-  // threads take consecutive rows so that the 2-byte gathers coalesce across the wave.
-  auto p_of = [&](int t) { return MODE == kBwdWeight ? t % BP : t >> 2; };
-  auto pk_of = [&](int t) { return MODE == kBwdWeight ? t / BP : t & 3; };
-  auto q_of = [&](int t) { return MODE == kBwdWeight ? t % BQ : t >> 2; };
-  auto qk_of = [&](int t) { return MODE == kBwdWeight ? t / BQ : t & 3; };
-
-  // Q-row pixel decode (forward, backward data), fixed across k steps
-  int q_img[NQ], q_y[NQ], q_x[NQ];
+  // rows past P repeat the last one (their results are not stored); pixels past Q read nothing
+  const uint16_t* wrow[TP];
 #pragma unroll
-  for (int i = 0; i < NQ; ++i) {
-    const int t = tid + i * kThreads;
-    const int64_t q = q0 + q_of(t);
-    q_img[i] = -1; q_y[i] = 0; q_x[i] = 0;
-    if (MODE != kBwdWeight && t < BQ * 4 && q < Q) {
-      const int hh = MODE == kFwd ? g.OH : g.H, ww = MODE == kFwd ? g.OW : g.W;
-      q_img[i] = int(q / (int64_t(hh) * ww));
-      const int r = int(q - int64_t(q_img[i]) * hh * ww);
-      q_y[i] = r / ww;
-      q_x[i] = r - q_y[i] * ww;
-    }
-  }
-
-  uint4 rP[NP], rQ[NQ];
-  auto load_step = [&](int64_t k0) {
+  for (int i = 0; i < TP; ++i)
+    wrow[i] = a.w + int64_t(min(p0 + 16 * i + row, P - 1)) * g.KS * g.KS * C + (ALIGNED ? 8 * kg : 0);
+  const uint16_t* src[TQ];                              // source pixel (sy, sx), where tap (0, 0) reads
+  int sy[TQ], sx[TQ];
+  {
+    const int per = ty.pixels * tx.pixels;
+    const int64_t q = q0 + row;
+    int b = quotient(q, per);
+    const int r = int(q - int64_t(b) * per);
+    int yc = r / tx.pixels, xc = r - yc * tx.pixels;
 #pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const int t = tid + i * kThreads;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (t < BP * 4) {
-        const int64_t p = p0 + p_of(t);
-        const int64_t k = k0 + pk_of(t) * 8;
-        if (MODE == kFwd) {
-          if (p < P && k < K) v = ld16(a.w + p * K + k);
-        } else if (MODE == kBwdData) {
-          if (p < P && k < K) v = ld16(a.wt + p * K + k);
-        } else if (p < P) {
-          const int tap = int(p / g.Cin), ci = int(p - int64_t(tap) * g.Cin);
-          const int kh = tap / g.KS, kw = tap - kh * g.KS;
-          uint16_t h[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            h[j] = 0;
-            if (k + j < kend) {
-              const int64_t off = in_offset(g, k + j, kh, kw, ci);
-              if (off >= 0) h[j] = a.x[off];
-            }
-          }
-          v = make_uint4(h[0] | (uint32_t(h[1]) << 16), h[2] | (uint32_t(h[3]) << 16),
-                         h[4] | (uint32_t(h[5]) << 16), h[6] | (uint32_t(h[7]) << 16));
-        }
+    for (int j = 0; j < TQ; ++j) {
+      const bool live = q + 16 * j < Q;
+      sy[j] = live ? yc * mul + ty.add : INT32_MIN / 2;
+      sx[j] = xc * mul + tx.add;
+      src[j] = a.src + ((int64_t(b) * SH + (live ? sy[j] : 0)) * SW + sx[j]) * C + (ALIGNED ? 8 * kg : 0);
+      if (tid < 16)
+        s_out[16 * j + row] = live ? ((int64_t(b) * DH + (FWD ? yc : yc * g.S + ry)) * DW + (FWD ? xc : xc * g.S + rx)) * P : -1;
+      xc += 16;
+      while (xc >= tx.pixels) {
+        xc -= tx.pixels;
+        if (++yc == ty.pixels) { yc = 0; ++b; }
       }
-      rP[i] = v;
     }
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      const int t = tid + i * kThreads;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (t < BQ * 4) {
-        const int64_t k = k0 + qk_of(t) * 8;
-        if (MODE == kFwd) {
-          if (q_img[i] >= 0 && k < K) {
-            const int tap = int(k / g.Cin), ci = int(k - int64_t(tap) * g.Cin);
-            const int kh = tap / g.KS, kw = tap - kh * g.KS;
-            const int ih = q_y[i] * g.S - g.PAD + kh, iw = q_x[i] * g.S - g.PAD + kw;
-            if (ih >= 0 && ih < g.H && iw >= 0 && iw < g.W)
-              v = ld16(a.x + ((int64_t(q_img[i]) * g.H + ih) * g.W + iw) * g.Cin + ci);
-          }
-        } else if (MODE == kBwdData) {
-          if (q_img[i] >= 0 && k < K) {
-            const int tap = int(k / g.Cout), co = int(k - int64_t(tap) * g.Cout);
-            const int kh = tap / g.KS, kw = tap - kh * g.KS;
-            const int ty = q_y[i] + g.PAD - kh, tx = q_x[i] + g.PAD - kw;
-            if (ty >= 0 && tx >= 0 && ty % g.S == 0 && tx % g.S == 0) {
-              const int oh = ty / g.S, ow = tx / g.S;
-              if (oh < g.OH && ow < g.OW)
-                v = ld16(a.dz + ((int64_t(q_img[i]) * g.OH + oh) * g.OW + ow) * g.Cout + co);
-            }
-          }
-        } else {
-          const int64_t q = q0 + q_of(t);
-          if (q < Q) {
-            uint16_t h[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) h[j] = (k + j < kend) ? a.dz[(k + j) * g.Cout + q] : uint16_t(0);
-            v = make_uint4(h[0] | (uint32_t(h[1]) << 16), h[2] | (uint32_t(h[3]) << 16),
-                           h[4] | (uint32_t(h[5]) << 16), h[6] | (uint32_t(h[7]) << 16));
-          }
-        }
-      }
-      rQ[i] = v;
-    }
-  };
+  }
 
   f32x4 acc[TP][TQ];
 #pragma unroll
@@ -214,138 +188,360 @@ __global__ __launch_bounds__(kThreads) void k_conv(ConvArgs a) {
 #pragma unroll
     for (int j = 0; j < TQ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int wp = wave & 1, wq = wave >> 1;
-  const int frow = lane & 15, fchunk = lane >> 4;
-
-  if (kbeg < kend) load_step(kbeg);
-  for (int64_t k0 = kbeg; k0 < kend; k0 += kBK) {
-    __syncthreads();
+  Words4 fa[NS][TP], fb[NS][TQ];
+  // tap (t, u) and channel c of a chunk; ALIGNED: uniform over the wave
+  auto load_tap = [&](int t, int u, unsigned c, bool live, Words4* va, Words4* vb) {
+    const int64_t wofs = int64_t((ty.k0 + kstep * t) * g.KS + tx.k0 + kstep * u) * C + c;
+    const int64_t sofs = (int64_t(dir * t) * SW + dir * u) * C + c;
 #pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const int t = tid + i * kThreads;
-      if (t < BP * 4) *reinterpret_cast<uint4*>(&sP[p_of(t) * kRow + pk_of(t) * 8]) = rP[i];
+    for (int i = 0; i < TP; ++i) {
+      va[i] = Words4{{0, 0, 0, 0}};
+      if (live) va[i] = *reinterpret_cast<const Words4*>(wrow[i] + wofs);
     }
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      const int t = tid + i * kThreads;
-      if (t < BQ * 4) *reinterpret_cast<uint4*>(&sQ[q_of(t) * kRow + qk_of(t) * 8]) = rQ[i];
-    }
-    __syncthreads();
-    if (k0 + kBK < kend) load_step(k0 + kBK);   // next step's global loads overlap the MFMAs
-    bf16x8 fa[TP], fb[TQ];
-#pragma unroll
-    for (int i = 0; i < TP; ++i)
-      fa[i] = *reinterpret_cast<const bf16x8*>(&sP[(wp * (BP / 2) + i * 16 + frow) * kRow + fchunk * 8]);
-#pragma unroll
-    for (int j = 0; j < TQ; ++j)
-      fb[j] = *reinterpret_cast<const bf16x8*>(&sQ[(wq * (BQ / 2) + j * 16 + frow) * kRow + fchunk * 8]);
-#pragma unroll
-    for (int i = 0; i < TP; ++i)
-#pragma unroll
-      for (int j = 0; j < TQ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-  }
-
-  // epilogue: lane holds D[p0 + .. + 4*(lane/16) + r][q0 + .. + lane%16], r = 0..3
-#pragma unroll
-  for (int i = 0; i < TP; ++i) {
-    const int64_t pb = p0 + wp * (BP / 2) + i * 16 + 4 * fchunk;
 #pragma unroll
     for (int j = 0; j < TQ; ++j) {
-      const int64_t q = q0 + wq * (BQ / 2) + j * 16 + frow;
-      if (q >= Q) continue;
-      float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-      if (MODE == kBwdWeight) {
-        float* o = static_cast<float*>(a.out) + (int64_t(blockIdx.z) * Q + q) * P + pb;
-        if (pb + 3 < P) {
-          *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-          for (int r = 0; r < 4; ++r)
-            if (pb + r < P) o[r] = v[r];
-        }
-        continue;
-      }
-      if (MODE == kFwd) {
+      vb[j] = Words4{{0, 0, 0, 0}};
+      if (live && (unsigned)(sy[j] + dir * t) < (unsigned)SH && (unsigned)(sx[j] + dir * u) < (unsigned)SW)
+        vb[j] = *reinterpret_cast<const Words4*>(src[j] + sofs);
+    }
+  };
+  const unsigned len = min((unsigned)NS, (steps + NW - 1) / NW);    // of a stretch
+  auto load_stretch = [&](unsigned first) {
+    if (ALIGNED) {
+      const unsigned per_tap = C8 / 4;
+      unsigned tap = first / per_tap, c = first - tap * per_tap;
+      int t = (int)(tap / (unsigned)max(tx.n, 1)), u = (int)tap - t * tx.n;
+      t = __builtin_amdgcn_readfirstlane(t);
+      u = __builtin_amdgcn_readfirstlane(u);
+      c = __builtin_amdgcn_readfirstlane(c);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if (pb + r < P) v[r] += a.bias[pb + r];
-          if (a.relu) v[r] = v[r] > 0.f ? v[r] : 0.f;
+      for (int k = 0; k < NS; ++k)
+        if (k < (int)len && first + k < steps) {
+          load_tap(t, u, 32 * c, true, fa[k], fb[k]);
+          if (++c == per_tap) {
+            c = 0;
+            if (++u == tx.n) { u = 0; ++t; }
+          }
         }
-      } else if (a.mask) {
+    } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (pb + r < P && !(bf2f(a.mask[q * P + pb + r]) > 0.f)) v[r] = 0.f;
+      for (int k = 0; k < NS; ++k)
+        if (k < (int)len && first + k < steps) {
+          const unsigned kc = (first + k) * 4 + kg;
+          const unsigned tap = kc / C8, c = (kc - tap * C8) * 8;
+          const int t = (int)(tap / (unsigned)tx.n), u = (int)tap - t * tx.n;
+          load_tap(t, u, c, kc < chunks, fa[k], fb[k]);
+        }
+    }
+  };
+  float* mine = tile + row * kRow + 4 * kg;
+  unsigned first = wave * len;                                      // this wave's stretch
+  load_stretch(first);
+  for (unsigned base = 0; base < steps; base += NW * len) {
+    for (int turn = 0; turn < NW && base + turn * len < steps; ++turn) {
+      if (turn == wave) {
+        if (NW > 1 && first > 0) {
+#pragma unroll
+          for (int i = 0; i < TP; ++i)
+#pragma unroll
+            for (int j = 0; j < TQ; ++j) acc[i][j] = *reinterpret_cast<const f32x4*>(mine + 16 * j * kRow + 16 * i);
+        }
+#pragma unroll
+        for (int k = 0; k < NS; ++k)
+          if (k < (int)len && first + k < steps) {
+#pragma unroll
+            for (int i = 0; i < TP; ++i)
+#pragma unroll
+              for (int j = 0; j < TQ; ++j) acc[i][j] = mfma(as_bf16x8(fa[k][i]), as_bf16x8(fb[k][j]), acc[i][j]);
+          }
+        if (NW > 1) {
+#pragma unroll
+          for (int i = 0; i < TP; ++i)
+#pragma unroll
+            for (int j = 0; j < TQ; ++j) *reinterpret_cast<f32x4*>(mine + 16 * j * kRow + 16 * i) = acc[i][j];
+        }
+        first += NW * len;
+        load_stretch(first);
       }
-      if (a.out_f32) {
-        float* o = static_cast<float*>(a.out) + q * P + pb;
-        for (int r = 0; r < 4; ++r)
-          if (pb + r < P) o[r] = v[r];
+      if (NW > 1) __syncthreads();
+    }
+  }
+  if (NW == 1 || steps == 0) {
+    if (wave == 0) {
+#pragma unroll
+      for (int i = 0; i < TP; ++i)
+#pragma unroll
+        for (int j = 0; j < TQ; ++j) *reinterpret_cast<f32x4*>(mine + 16 * j * kRow + 16 * i) = acc[i][j];
+    }
+    __syncthreads();
+  }
+
+  // the epilogue: 8 consecutive p of one q per thread
+  for (int e = tid; e < BQ * (BP / 8); e += 64 * NW) {
+    const int ql = e / (BP / 8), pl = (e - ql * (BP / 8)) * 8;
+    const int64_t so = s_out[ql];
+    const int pb = p0 + pl;
+    if (so < 0 || pb >= P) continue;                    // P is a multiple of 8
+    float v[8];
+    const float* t0 = tile + ql * kRow + pl;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = t0[k];
+    const int64_t o = so + pb;
+    if (FWD) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        v[k] += a.bias[pb + k];
+        if (a.relu) v[k] = v[k] > 0.f ? v[k] : 0.f;
+      }
+    } else if (a.mask) {
+      uint16_t m[8];
+      __builtin_memcpy(m, a.mask + o, 16);
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (!(bf2f(m[k]) > 0.f)) v[k] = 0.f;
+    }
+    if (FWD && a.out_f32) {
+      float* d = static_cast<float*>(a.out) + o;
+      if (a.wide) {
+        *reinterpret_cast<float4*>(d) = make_float4(v[0], v[1], v[2], v[3]);
+        *reinterpret_cast<float4*>(d + 4) = make_float4(v[4], v[5], v[6], v[7]);
       } else {
-        uint16_t* o = static_cast<uint16_t*>(a.out) + q * P + pb;
-        if (pb + 3 < P) {
-          *reinterpret_cast<uint2*>(o) = make_uint2(f2bf(v[0]) | (uint32_t(f2bf(v[1])) << 16),
-                                                    f2bf(v[2]) | (uint32_t(f2bf(v[3])) << 16));
-        } else {
-          for (int r = 0; r < 4; ++r)
-            if (pb + r < P) o[r] = f2bf(v[r]);
-        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) d[k] = v[k];
+      }
+      continue;
+    }
+    uint16_t* d = static_cast<uint16_t*>(a.out) + o;
+    bf16x8 h;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) h[k] = static_cast<__bf16>(v[k]);         // round to nearest even
+    if (a.wide) *reinterpret_cast<bf16x8*>(d) = h;
+    else __builtin_memcpy(d, &h, 16);
+  }
+}
+
+// ---- backward weight -----------------------------------------------------------------------
+// The reduction runs over pixels, which are strided in NHWC, while an MFMA operand wants 8
+// consecutive k in a lane.  Each lane loads 8 pixels x 8 channels of x (8 pixels x NB channels of
+// dz) with one vector load per pixel and transposes them in registers, one byte permute per pair
+// of pixels and channel.  Fragment j then holds channel j of every lane's chunk: rows 8 r + j of
+// the 128-row P tile (columns NB n + j of the 32-column Q tile, NB = 2), a fixed permutation that
+// the epilogue undoes with 32-byte stores.  2-byte gathers into LDS took 385 us for the network's
+// layers of 16 images, and the bias sums, formed here with a row of ones, 83 us of their own.
+constexpr int kWP = 128, kWQ = 32;       // rows and columns of a tile; 128 x 64 halves the waves per SIMD: 131 us
+                                         // against 111 for the network's seven layers at 16 images
+constexpr int kWWaves = 4;               // waves of a workgroup, splitting its pixels
+constexpr int64_t kWeightBlocks = 512, kWeightSteps = 4;   // weight_split
+
+struct WeightArgs {
+  ConvGeom g;
+  const uint16_t* x;       // [B][H][W][Cin]
+  const uint16_t* dz;      // [B][OH][OW][Cout]
+  float* dw;               // splits > 1: partials [splits][Cout][P]; else the gradient itself
+  float* db;               // [splits][Cout] or null
+  int64_t per;             // pixels per split (a multiple of 32 kWWaves)
+  int wide;                // dw is 16-byte aligned
+};
+
+__device__ __forceinline__ uint32_t lo_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
+__device__ __forceinline__ uint32_t hi_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+
+__global__ __launch_bounds__(64 * kWWaves) void k_conv_weight(WeightArgs a) {
+  constexpr int NB = kWQ / 16, kVals = 8 * NB * 4 + NB;   // per lane: 8 x NB fragments, and the bias column sums
+  __shared__ float red[kWWaves / 2][kVals][64];
+  const ConvGeom g = a.g;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = lane & 15, kg = lane >> 4;
+  const int P = g.KS * g.KS * g.Cin, Q = g.Cout;
+  const int64_t K = int64_t(g.B) * g.OH * g.OW;
+  const int q0 = blockIdx.x * kWQ, p0 = blockIdx.y * kWP;
+  const bool bias = a.db && blockIdx.y == 0;
+  // this lane's chunk of 8 rows (one tap) and its NB columns; chunks past the end load nothing
+  const int pc = p0 + 8 * row, qc = q0 + NB * row;
+  const bool p_live = pc < P, q_live = qc < Q;
+  const int tap = p_live ? pc / g.Cin : 0, ci = p_live ? pc - tap * g.Cin : 0;
+  const int kh = tap / g.KS, kw = tap - kh * g.KS;
+  const int64_t beg = int64_t(blockIdx.z) * a.per;
+  const int64_t end = beg + a.per < K ? beg + a.per : K;
+
+  uint32_t rx[8][4], rz[8][NB / 2];
+  const int64_t xstep = int64_t(g.S) * g.Cin;
+  const bool whole = g.OW % 8 == 0;          // a lane's 8 pixels lie in one row
+  auto load = [&](int64_t k0) {
+    int64_t k = k0 + 8 * kg;
+    const int ohw = g.OH * g.OW;
+    int b = quotient(k, ohw);
+    const int r = int(k - int64_t(b) * ohw);
+    int oh = r / g.OW, ow = r - oh * g.OW;
+    const uint16_t* px = a.x + ((int64_t(b) * g.H + oh * g.S - g.PAD + kh) * g.W + ow * g.S - g.PAD + kw) * g.Cin + ci;
+    const uint16_t* pz = a.dz + k * g.Cout + qc;
+    const int live = int(end - k < 8 ? end - k : 8);        // pixels of this lane before the end
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) rx[i][c] = 0;
+#pragma unroll
+      for (int c = 0; c < NB / 2; ++c) rz[i][c] = 0;
+      if (i < live) {
+        const int ih = oh * g.S - g.PAD + kh, iw = ow * g.S - g.PAD + kw;
+        if (p_live && (unsigned)ih < (unsigned)g.H && (unsigned)iw < (unsigned)g.W) __builtin_memcpy(rx[i], px, 16);
+        if (q_live) __builtin_memcpy(rz[i], pz + i * int64_t(g.Cout), 2 * NB);
+      }
+      ++ow;
+      px += xstep;
+      if (!whole && ow == g.OW) {
+        ow = 0;
+        if (++oh == g.OH) { oh = 0; ++b; }
+        px = a.x + ((int64_t(b) * g.H + oh * g.S - g.PAD + kh) * g.W - g.PAD + kw) * g.Cin + ci;
+      }
+    }
+  };
+
+  f32x4 acc[8][NB], accb[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    accb[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const bf16x8 ones = as_bf16x8(Words4{{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u}});
+  int64_t k0 = beg + 32 * wave;
+  if (k0 < end) load(k0);
+  for (; k0 < end; k0 += 32 * kWWaves) {
+    bf16x8 fx[8], fz[NB];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      Words4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v.w[i] = c & 1 ? hi_halves(rx[2 * i][c / 2], rx[2 * i + 1][c / 2])
+                                                 : lo_halves(rx[2 * i][c / 2], rx[2 * i + 1][c / 2]);
+      fx[c] = as_bf16x8(v);
+    }
+#pragma unroll
+    for (int c = 0; c < NB; ++c) {
+      Words4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v.w[i] = c & 1 ? hi_halves(rz[2 * i][c / 2], rz[2 * i + 1][c / 2])
+                                                 : lo_halves(rz[2 * i][c / 2], rz[2 * i + 1][c / 2]);
+      fz[c] = as_bf16x8(v);
+    }
+    if (k0 + 32 * kWWaves < end) load(k0 + 32 * kWWaves);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[i][j] = mfma(fx[i], fz[j], acc[i][j]);
+    if (bias) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) accb[j] = mfma(ones, fz[j], accb[j]);
+    }
+  }
+
+  // sum the waves pairwise through LDS: (0 + 2), (1 + 3), then 0 + 1
+#pragma unroll
+  for (int half = kWWaves / 2; half >= 1; half >>= 1) {
+    __syncthreads();
+    if (wave >= half && wave < 2 * half) {
+      float(*d)[64] = red[wave - half];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) d[(i * NB + j) * 4 + r][lane] = acc[i][j][r];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) d[32 * NB + j][lane] = accb[j][0];
+    }
+    __syncthreads();
+    if (wave < half) {
+      const float(*d)[64] = red[wave];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[i][j][r] += d[(i * NB + j) * 4 + r][lane];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) accb[j][0] += d[32 * NB + j][lane];
+    }
+  }
+  if (wave != 0 || !q_live) return;
+  // accumulator r of fragment pair (i, j): p = p0 + 8 (4 kg + r) + i, q = q0 + NB row + j
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int q = qc + j;
+    if (q >= Q) continue;
+    if (bias && kg == 0) a.db[int64_t(blockIdx.z) * Q + q] = accb[j][0];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int p = p0 + 8 * (4 * kg + r);
+      if (p >= P) continue;
+      float* o = a.dw + (int64_t(blockIdx.z) * Q + q) * P + p;
+      if (a.wide) {
+        *reinterpret_cast<float4*>(o) = make_float4(acc[0][j][r], acc[1][j][r], acc[2][j][r], acc[3][j][r]);
+        *reinterpret_cast<float4*>(o + 4) = make_float4(acc[4][j][r], acc[5][j][r], acc[6][j][r], acc[7][j][r]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = acc[i][j][r];
       }
     }
   }
 }
 
-// out[i] = sum_s part[s][i], deterministic.  Block: 64 consecutive outputs x 4 split lanes;
-// each lane sums every 4th split, then the four partial sums are added in fixed order.
-__global__ __launch_bounds__(256) void k_split_sum(const float* __restrict__ part, int splits, int64_t n,
-                                                   float* __restrict__ out) {
-  __shared__ float red[4][64];
-  const int64_t i = int64_t(blockIdx.x) * 64 + (threadIdx.x & 63);
+// dw[i] = sum_s part[s][i] and db likewise, deterministic.  Block: 64 consecutive outputs x 16
+// split lanes; each lane sums every 16th split, then the 16 partial sums are added in order.
+constexpr int kSumLanes = 16;
+__global__ __launch_bounds__(64 * kSumLanes) void k_split_sum(const float* __restrict__ part, const float* __restrict__ bpart,
+                                                              int splits, int64_t n, int nb, float* __restrict__ out,
+                                                              float* __restrict__ bout) {
+  __shared__ float red[kSumLanes][64];
+  const int64_t wblocks = (n + 63) / 64;
+  const bool is_bias = (int64_t)blockIdx.x >= wblocks;
+  const float* src = is_bias ? bpart : part;
+  float* dst = is_bias ? bout : out;
+  const int64_t m = is_bias ? nb : n;
+  const int64_t i = (int64_t(blockIdx.x) - (is_bias ? wblocks : 0)) * 64 + (threadIdx.x & 63);
   const int r = threadIdx.x >> 6;
   float s = 0.f;
-  if (i < n)
-    for (int k = r; k < splits; k += 4) s += part[int64_t(k) * n + i];
+  if (i < m) {
+#pragma unroll 4
+    for (int k = r; k < splits; k += kSumLanes) s += src[int64_t(k) * m + i];
+  }
   red[r][threadIdx.x & 63] = s;
   __syncthreads();
-  if (r == 0 && i < n) out[i] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
-}
-
-// Bias gradient partials: part[split][c] = sum over the split's pixels of dz[pix][c].
-// Block: 64 channels x 4 pixel lanes; grid (ceil(C/64), splits).  Each lane keeps four
-// independent running sums so that four loads are in flight.
-__global__ __launch_bounds__(256) void k_bias_partial(const uint16_t* __restrict__ dz, int64_t pixels, int C,
-                                                      int64_t per_split, float* __restrict__ part) {
-  __shared__ float red[4][64];
-  const int c = blockIdx.x * 64 + (threadIdx.x & 63), r = threadIdx.x >> 6;
-  const int64_t beg = int64_t(blockIdx.y) * per_split;
-  const int64_t end = beg + per_split < pixels ? beg + per_split : pixels;
-  float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-  if (c < C) {
-    int64_t p = beg + r;
-    for (; p + 12 < end; p += 16) {
-      s0 += bf2f(dz[p * C + c]);
-      s1 += bf2f(dz[(p + 4) * C + c]);
-      s2 += bf2f(dz[(p + 8) * C + c]);
-      s3 += bf2f(dz[(p + 12) * C + c]);
-    }
-    for (; p < end; p += 4) s0 += bf2f(dz[p * C + c]);
+  if (r == 0 && i < m) {
+    float t = 0.f;
+#pragma unroll
+    for (int k = 0; k < kSumLanes; ++k) t += red[k][threadIdx.x];
+    dst[i] = t;
   }
-  red[r][threadIdx.x & 63] = (s0 + s1) + (s2 + s3);
-  __syncthreads();
-  if (r == 0 && c < C)
-    part[int64_t(blockIdx.y) * C + c] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
-// fp32 master weights [Cout][T][Cin] -> bf16 copy and bf16 transpose [Cin][T][Cout]
-__global__ void k_prepare_weights(const float* __restrict__ w, int Cout, int T, int Cin, uint16_t* __restrict__ wb,
-                                  uint16_t* __restrict__ wt) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+// fp32 master weights [Cout][T][Cin] -> bf16 copy and bf16 transpose [Cin][T][Cout], for up to
+// kPrepareLayers layers in one launch (a launch of its own per layer took 4 us each, 5 to 7 layers
+// of them idle): layer l owns blocks [start[l], start[l + 1]).
+constexpr int kPrepareLayers = 16;
+struct PrepareArgs {
+  const float* w[kPrepareLayers];
+  uint16_t* wb[kPrepareLayers];
+  uint16_t* wt[kPrepareLayers];
+  int cout[kPrepareLayers], taps[kPrepareLayers], cin[kPrepareLayers];
+  unsigned start[kPrepareLayers + 1];
+  int n;
+};
+
+__global__ void k_prepare_weights(PrepareArgs a) {
+  int l = 0;
+  while (l + 1 < a.n && blockIdx.x >= a.start[l + 1]) ++l;
+  const int Cout = a.cout[l], T = a.taps[l], Cin = a.cin[l];
+  const int64_t i = int64_t(blockIdx.x - a.start[l]) * blockDim.x + threadIdx.x;
   const int64_t n = int64_t(Cout) * T * Cin;
   if (i >= n) return;
   const int ci = int(i % Cin);
   const int64_t r = i / Cin;
   const int t = int(r % T), co = int(r / T);
-  const uint16_t h = f2bf(w[i]);
-  wb[i] = h;
-  if (wt) wt[(int64_t(ci) * T + t) * Cout + co] = h;
+  const uint16_t h = f2bf(a.w[l][i]);
+  a.wb[l][i] = h;
+  if (a.wt[l]) a.wt[l][(int64_t(ci) * T + t) * Cout + co] = h;
 }
 
 // Renders [B][V][h][w][3] fp32 -> NHWC8 bf16 mosaic [B][rows*h/d][cols*w/d][8]: view v at tile
@@ -430,43 +626,63 @@ int hip_status(const char* what) {
   return 0;
 }
 
-template <int MODE, int BP, int BQ>
-void launch(const ConvArgs& a, int splits, hipStream_t s) {
-  int64_t P, Q, K;
-  gemm_dims(MODE, a.g, P, Q, K);
-  dim3 grid(unsigned((Q + BQ - 1) / BQ), unsigned((P + BP - 1) / BP), unsigned(splits));
-  hipLaunchKernelGGL((k_conv<MODE, BP, BQ>), grid, dim3(kThreads), 0, s, a);
+template <bool FWD, int TP, int TQ, int NW, int NS>
+int launch(ConvArgs a, hipStream_t s, const char* what) {
+  const ConvGeom& g = a.g;
+  const int cy = FWD ? 1 : (g.S < g.H ? g.S : g.H), cx = FWD ? 1 : (g.S < g.W ? g.S : g.W);
+  // the class of residue 0 has the most pixels
+  const int64_t Q = FWD ? int64_t(g.B) * g.OH * g.OW
+                        : int64_t(g.B) * ((g.H + g.S - 1) / g.S) * ((g.W + g.S - 1) / g.S);
+  const int P = FWD ? g.Cout : g.Cin;
+  a.ptiles = (P + 16 * TP - 1) / (16 * TP);
+  const int64_t qtiles = (Q + 16 * TQ - 1) / (16 * TQ);
+  const int64_t blocks = qtiles * a.ptiles * cy * cx;
+  if (blocks > INT32_MAX) return gvv::set_last_error(std::string(what) + ": too many output tiles");
+  a.qtiles = int(qtiles);
+  a.classes_x = cx;
+  if ((FWD ? g.Cin : g.Cout) % 32 == 0)
+    hipLaunchKernelGGL((k_conv<FWD, true, TP, TQ, NW, NS>), dim3(unsigned(blocks)), dim3(64 * NW), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_conv<FWD, false, TP, TQ, NW, NS>), dim3(unsigned(blocks)), dim3(64 * NW), 0, s, a);
+  return hip_status(what);
 }
 
-// Tile choice: narrow P (32 channels) takes 32 x 128; otherwise 64 x 128 when Q is large
-// enough to fill the chip, else 64 x 64.
-template <int MODE>
-void launch_tiled(const ConvArgs& a, int splits, hipStream_t s) {
-  int64_t P, Q, K;
-  gemm_dims(MODE, a.g, P, Q, K);
-  if (P <= 32) launch<MODE, 32, 128>(a, splits, s);
-  else if (Q >= 64 * 1024) launch<MODE, 64, 128>(a, splits, s);
-  else launch<MODE, 64, 64>(a, splits, s);
+// Tile choice: the largest tile that still gives the chip's 256 CUs a workgroup each, as a larger
+// tile reads its operands fewer times.  With 1024 tiles and more, one wave per tile fills the chip
+// and passes no accumulators (backward data of the 64-channel layer at 16 images: 29 us against 38
+// with four waves, of the 128-channel layer 24 against 28); with fewer, the stretches of the
+// reduction are loaded side by side (the 4096-deep head: 15 us, one wave 75).  Tiles of 32 x 128 and
+// 64 x 128 were no faster (30 and 30 us for those two).
+template <bool FWD>
+int launch_conv(const ConvArgs& a, hipStream_t s, const char* what) {
+  const ConvGeom& g = a.g;
+  const int64_t Q = FWD ? int64_t(g.B) * g.OH * g.OW : int64_t(g.B) * g.H * g.W;
+  const int64_t P = FWD ? g.Cout : g.Cin;
+  const int taps = FWD ? g.KS : (g.KS + g.S - 1) / g.S;            // of one axis, at most
+  const int64_t steps = (int64_t(taps) * taps * (FWD ? g.Cin : g.Cout) + 31) / 32;
+  auto tiles = [&](int bp, int bq) { return ((P + bp - 1) / bp) * ((Q + bq - 1) / bq); };
+  if (P <= 32 && tiles(32, 64) >= 1024) return launch<FWD, 2, 4, 1, 2>(a, s, what);
+  if (P <= 32 && tiles(32, 64) >= 256) return launch<FWD, 2, 4, 4, 3>(a, s, what);
+  if (P > 32 && tiles(64, 64) >= 1024) return launch<FWD, 4, 4, 1, 2>(a, s, what);
+  if (P > 32 && tiles(64, 64) >= 256) return launch<FWD, 4, 4, 4, 3>(a, s, what);
+  if (P > 16 && tiles(32, 32) >= 256) return launch<FWD, 2, 2, 8, 5>(a, s, what);
+  return steps < 16 ? launch<FWD, 1, 1, 4, 4>(a, s, what) : launch<FWD, 1, 1, 16, 8>(a, s, what);
 }
 
-// Split of the weight-gradient reduction: enough (P, Q) tiles x splits to fill 256 CUs a few
-// times over, each split at least 8 k-steps (256 pixels) and at most 1024 splits; k_split_sum
-// reduces the partials in parallel over outputs and splits.
+// Split of the weight-gradient reduction over workgroups: enough workgroups for the chip
+// (about 512 of four waves), each with at least 4 steps of 32 pixels per wave, which keeps the
+// partial sums (read once more by k_split_sum) a small share of the traffic.
 void weight_split(const ConvGeom& g, int& splits, int64_t& per) {
-  int64_t P, Q, K;
-  gemm_dims(kBwdWeight, g, P, Q, K);
-  const int BP = P <= 32 ? 32 : 64, BQ = P <= 32 ? 128 : (Q >= 64 * 1024 ? 128 : 64);
-  const int64_t tiles = ((P + BP - 1) / BP) * ((Q + BQ - 1) / BQ);
-  const int64_t steps = (K + kBK - 1) / kBK;
-  int64_t want = (2048 + tiles - 1) / tiles;
-  if (want > steps / 8) want = steps / 8;
-  if (want > 1024) want = 1024;
+  const int64_t P = int64_t(g.KS) * g.KS * g.Cin, K = int64_t(g.B) * g.OH * g.OW;
+  const int64_t tiles = ((P + kWP - 1) / kWP) * ((g.Cout + kWQ - 1) / kWQ);
+  constexpr int64_t unit = 32 * kWWaves;               // pixels of one step of every wave
+  const int64_t steps = (K + unit - 1) / unit;
+  int64_t want = (kWeightBlocks + tiles - 1) / tiles;
+  if (want > steps / kWeightSteps) want = steps / kWeightSteps;
   if (want < 1) want = 1;
-  per = ((steps + want - 1) / want) * kBK;
+  per = ((steps + want - 1) / want) * unit;
   splits = int((K + per - 1) / per);
 }
-
-constexpr int64_t kBiasPer = 1024;   // pixels per bias-gradient partial
 
 }  // namespace
 
@@ -487,14 +703,14 @@ int gvv_conv_forward(int32_t B, int32_t H, int32_t W, int32_t Cin, int32_t Cout,
   if (!aligned16(x) || !aligned16(w)) return gvv::set_last_error("conv forward: x and w must be 16-byte aligned");
   ConvArgs a{};
   a.g = g;
-  a.x = static_cast<const uint16_t*>(x);
+  a.src = static_cast<const uint16_t*>(x);
   a.w = static_cast<const uint16_t*>(w);
   a.bias = bias;
   a.out = y;
   a.out_f32 = y_f32 ? 1 : 0;
   a.relu = relu ? 1 : 0;
-  launch_tiled<kFwd>(a, 1, static_cast<hipStream_t>(stream));
-  return hip_status("conv forward");
+  a.wide = aligned16(y) ? 1 : 0;
+  return launch_conv<true>(a, static_cast<hipStream_t>(stream), "conv forward");
 }
 
 int gvv_conv_backward_data(int32_t B, int32_t H, int32_t W, int32_t Cin, int32_t Cout, int32_t ks, int32_t stride,
@@ -506,12 +722,12 @@ int gvv_conv_backward_data(int32_t B, int32_t H, int32_t W, int32_t Cin, int32_t
   if (!aligned16(dz) || !aligned16(wt)) return gvv::set_last_error("conv backward data: dz and wt must be 16-byte aligned");
   ConvArgs a{};
   a.g = g;
-  a.dz = static_cast<const uint16_t*>(dz);
-  a.wt = static_cast<const uint16_t*>(wt);
+  a.src = static_cast<const uint16_t*>(dz);
+  a.w = static_cast<const uint16_t*>(wt);
   a.mask = static_cast<const uint16_t*>(x_mask);
   a.out = dx;
-  launch_tiled<kBwdData>(a, 1, static_cast<hipStream_t>(stream));
-  return hip_status("conv backward data");
+  a.wide = aligned16(dx) ? 1 : 0;
+  return launch_conv<false>(a, static_cast<hipStream_t>(stream), "conv backward data");
 }
 
 int64_t gvv_conv_workspace_floats(int32_t B, int32_t H, int32_t W, int32_t Cin, int32_t Cout, int32_t ks,
@@ -522,9 +738,7 @@ int64_t gvv_conv_workspace_floats(int32_t B, int32_t H, int32_t W, int32_t Cin, 
   int splits;
   int64_t per;
   weight_split(g, splits, per);
-  const int64_t pixels = int64_t(B) * g.OH * g.OW;
-  const int64_t bsplits = (pixels + kBiasPer - 1) / kBiasPer;
-  return int64_t(splits) * Cout * ks * ks * Cin + bsplits * Cout;
+  return int64_t(splits) * Cout * ks * ks * Cin + int64_t(splits) * Cout;
 }
 
 int gvv_conv_backward_weight(int32_t B, int32_t H, int32_t W, int32_t Cin, int32_t Cout, int32_t ks, int32_t stride,
@@ -542,36 +756,58 @@ int gvv_conv_backward_weight(int32_t B, int32_t H, int32_t W, int32_t Cin, int32
   int splits;
   int64_t per;
   weight_split(g, splits, per);
-  ConvArgs a{};
+  const int64_t P = int64_t(ks) * ks * Cin, n = P * Cout;
+  const int64_t ptiles = (P + kWP - 1) / kWP;
+  if (P > INT32_MAX - kWP || ptiles > 65535 || splits > 65535)
+    return gvv::set_last_error("conv backward weight: too many weight rows");
+  WeightArgs a{};
   a.g = g;
   a.x = static_cast<const uint16_t*>(x);
   a.dz = static_cast<const uint16_t*>(dz);
-  a.out = workspace;
-  a.out_f32 = 1;
-  a.k_per_split = per;
-  launch_tiled<kBwdWeight>(a, splits, s);
-  const int64_t n = int64_t(Cout) * ks * ks * Cin;
-  hipLaunchKernelGGL(k_split_sum, dim3(unsigned((n + 63) / 64)), dim3(256), 0, s, workspace, splits, n, dw);
-  if (db) {
-    const int64_t pixels = int64_t(B) * g.OH * g.OW;
-    const int bsplits = int((pixels + kBiasPer - 1) / kBiasPer);
-    float* bpart = workspace + int64_t(splits) * n;
-    hipLaunchKernelGGL(k_bias_partial, dim3(unsigned((Cout + 63) / 64), unsigned(bsplits)), dim3(256), 0, s,
-                       static_cast<const uint16_t*>(dz), pixels, Cout, kBiasPer, bpart);
-    hipLaunchKernelGGL(k_split_sum, dim3(unsigned((Cout + 63) / 64)), dim3(256), 0, s, bpart, bsplits,
-                       int64_t(Cout), db);
+  a.dw = splits > 1 ? workspace : dw;
+  a.db = !db ? nullptr : splits > 1 ? workspace + int64_t(splits) * n : db;
+  a.per = per;
+  a.wide = aligned16(a.dw) ? 1 : 0;
+  const dim3 grid(unsigned((Cout + kWQ - 1) / kWQ), unsigned(ptiles), unsigned(splits));
+  hipLaunchKernelGGL(k_conv_weight, grid, dim3(64 * kWWaves), 0, s, a);
+  if (splits > 1) {
+    const unsigned blocks = unsigned((n + 63) / 64 + (db ? (Cout + 63) / 64 : 0));
+    hipLaunchKernelGGL(k_split_sum, dim3(blocks), dim3(64 * kSumLanes), 0, s, workspace, a.db, splits, n, Cout, dw, db);
   }
   return hip_status("conv backward weight");
 }
 
+int gvv_conv_prepare_weights_layers(int32_t n, const int32_t* Cout, const int32_t* taps, const int32_t* Cin,
+                                    const float* const* w, void* const* w_bf16, void* const* wt_bf16, void* stream) {
+  if (n <= 0 || !Cout || !taps || !Cin || !w || !w_bf16 || !wt_bf16)
+    return gvv::set_last_error("prepare weights: need at least one layer and its tables");
+  for (int32_t l = 0; l < n; ++l) {
+    if (Cout[l] <= 0 || taps[l] <= 0 || Cin[l] <= 0) return gvv::set_last_error("prepare weights: sizes must be positive");
+    if (!w[l] || !w_bf16[l]) return gvv::set_last_error("prepare weights: null pointer");
+  }
+  for (int32_t l0 = 0; l0 < n; l0 += kPrepareLayers) {
+    PrepareArgs a{};
+    int64_t blocks = 0;
+    for (int32_t l = l0; l < n && l < l0 + kPrepareLayers; ++l) {
+      const int k = l - l0;
+      a.w[k] = w[l];
+      a.wb[k] = static_cast<uint16_t*>(w_bf16[l]);
+      a.wt[k] = static_cast<uint16_t*>(wt_bf16[l]);
+      a.cout[k] = Cout[l]; a.taps[k] = taps[l]; a.cin[k] = Cin[l];
+      a.start[k] = unsigned(blocks);
+      blocks += (int64_t(Cout[l]) * taps[l] * Cin[l] + 255) / 256;
+      if (blocks > INT32_MAX) return gvv::set_last_error("prepare weights: too many weights");
+      a.n = k + 1;
+      a.start[k + 1] = unsigned(blocks);
+    }
+    hipLaunchKernelGGL(k_prepare_weights, dim3(unsigned(blocks)), dim3(256), 0, static_cast<hipStream_t>(stream), a);
+  }
+  return hip_status("prepare weights");
+}
+
 int gvv_conv_prepare_weights(int32_t Cout, int32_t taps, int32_t Cin, const float* w, void* w_bf16, void* wt_bf16,
                              void* stream) {
-  if (Cout <= 0 || taps <= 0 || Cin <= 0) return gvv::set_last_error("prepare weights: sizes must be positive");
-  if (!w || !w_bf16) return gvv::set_last_error("prepare weights: null pointer");
-  const int64_t n = int64_t(Cout) * taps * Cin;
-  hipLaunchKernelGGL(k_prepare_weights, dim3(unsigned((n + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream),
-                     w, Cout, taps, Cin, static_cast<uint16_t*>(w_bf16), static_cast<uint16_t*>(wt_bf16));
-  return hip_status("prepare weights");
+  return gvv_conv_prepare_weights_layers(1, &Cout, &taps, &Cin, &w, &w_bf16, &wt_bf16, stream);
 }
 
 int gvv_pack_mosaic(const float* render, int32_t B, int32_t V, int32_t h, int32_t w, int32_t cols, int32_t down,

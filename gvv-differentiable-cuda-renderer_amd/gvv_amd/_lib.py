@@ -18,7 +18,8 @@ EXPORTS = ("gvv_last_error", "gvv_version", "gvv_create", "gvv_destroy", "gvv_fo
            "gvv_set_depth_pass", "gvv_get_depth_pass",
            "gvv_calibrate_atomics",
            "gvv_conv_out_size", "gvv_conv_forward", "gvv_conv_backward_data", "gvv_conv_workspace_floats",
-           "gvv_conv_backward_weight", "gvv_conv_prepare_weights", "gvv_pack_mosaic",
+           "gvv_conv_backward_weight", "gvv_conv_prepare_weights", "gvv_conv_prepare_weights_layers",
+           "gvv_pack_mosaic",
            "gvv_multi_create", "gvv_multi_destroy", "gvv_multi_run", "gvv_multi_use_graph", "gvv_multi_autotune",
            "gvv_multi_set_batched", "gvv_multi_set_tuning",
            "gvv_multi_tuning",
@@ -80,6 +81,8 @@ def load():
     L.gvv_conv_backward_weight.restype = ctypes.c_int
     L.gvv_conv_prepare_weights.argtypes = [i32, i32, i32, P, P, P, P]
     L.gvv_conv_prepare_weights.restype = ctypes.c_int
+    L.gvv_conv_prepare_weights_layers.argtypes = [i32, P, P, P, P, P, P, P]
+    L.gvv_conv_prepare_weights_layers.restype = ctypes.c_int
     L.gvv_pack_mosaic.argtypes = [P, i32, i32, i32, i32, i32, i32, i32, P, P]
     L.gvv_pack_mosaic.restype = ctypes.c_int
     L.gvv_multi_create.argtypes = [P, i32, i32, i32, ctypes.POINTER(P)]

@@ -131,10 +131,13 @@ class ProposalNet:
 
     def refresh(self):
         """Re-derive the bf16 (and transposed bf16) weight copies from the FP32 masters."""
-        s = _stream()
-        for l, w, wb, wt in zip(self.layers, self.w, self.wb, self.wt):
-            _lib.check(self.L.gvv_conv_prepare_weights(l.Cout, l.ks * l.ks, l.Cin, _ptr(w), _ptr(wb), _ptr(wt), s),
-                       "gvv_conv_prepare_weights")
+        n = len(self.layers)
+        ints, ptrs = ctypes.c_int32 * n, ctypes.c_void_p * n
+        _lib.check(self.L.gvv_conv_prepare_weights_layers(
+            n, ints(*(l.Cout for l in self.layers)), ints(*(l.ks * l.ks for l in self.layers)),
+            ints(*(l.Cin for l in self.layers)), ptrs(*(w.data_ptr() for w in self.w)),
+            ptrs(*(w.data_ptr() for w in self.wb)), ptrs(*(w.data_ptr() for w in self.wt)), _stream()),
+            "gvv_conv_prepare_weights_layers")
 
     def state_dict(self):
         return {f"w{i}": w.detach().cpu() for i, w in enumerate(self.w)} | \

@@ -51,6 +51,10 @@ int gvv_conv_backward_weight(int32_t B, int32_t H, int32_t W, int32_t Cin, int32
 int gvv_conv_prepare_weights(int32_t Cout, int32_t taps, int32_t Cin, const float* w, void* w_bf16, void* wt_bf16,
                              void* stream);
 
+/* The same for n layers in one launch (host tables of n entries; wt_bf16 entries may be NULL). */
+int gvv_conv_prepare_weights_layers(int32_t n, const int32_t* Cout, const int32_t* taps, const int32_t* Cin,
+                                    const float* const* w, void* const* w_bf16, void* const* wt_bf16, void* stream);
+
 /* fp32 renders [B][V][h][w][3] -> bf16 NHWC8 mosaic [B][ceil(V/cols)*h/down][cols*w/down][8]:
  * view v at tile (v / cols, v % cols), each pixel the mean of a down x down block of the view.
  * features 0: channels 0..2 RGB, 3..7 zero.  features 1: channels 0..2 RGB - 0.5, 3 the covered
