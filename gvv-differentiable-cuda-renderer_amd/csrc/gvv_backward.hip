@@ -180,7 +180,7 @@ __device__ __forceinline__ void pixel_terms(const BackwardArgs& a, const Camera&
   }
   const V3 un = n0 * abc.x + n1 * abc.y + n2 * abc.z;
   const float unl = length(un);
-  V3 n = un / unl;         // IEEE division: the flip decision below is part of the binary32 contract
+  V3 n = over(un, unl);    // correctly rounded: the flip decision below is part of the binary32 contract
   const bool flipped = dot(n, d) > 0.f;
   if (flipped) n = -n;
 

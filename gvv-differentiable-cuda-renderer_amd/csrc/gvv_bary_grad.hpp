@@ -144,11 +144,13 @@ GVV_HD BaryGradSetup bary_grad_pixel(const BaryFace& f, V3 o, V3 d, V3 v0) {
   nl = nl + (dot(wl, g.N) + dot(wh, Nl));
   dot2(d, g.N, dh, dl);
   dl = dl + dot(d, Nl);
-  // t = (nh + nl) / (dh + dl) as th + tl
-  const float th = nh / dh;
+  // t = (nh + nl) / (dh + dl) as th + tl: th may be any value within a few ulp of nh / dh, as tl is
+  // formed from its exact residual, so both take the reciprocal of dh
+  const float rd = rcp_rn(dh);
+  const float th = nh * rd;
   float ph, pl;
   two_prod(th, dh, ph, pl);
-  const float tl = (((nh - ph) - pl) + (nl - th * dl)) / dh;
+  const float tl = (((nh - ph) - pl) + (nl - th * dl)) * rd;
   // q0 = t d - w, component by component from the exact residuals
   float q[3];
   const float dv[3] = {d.x, d.y, d.z}, whv[3] = {wh.x, wh.y, wh.z}, wlv[3] = {wl.x, wl.y, wl.z};

@@ -182,15 +182,18 @@ __global__ void __launch_bounds__(256) k_vertices_multi(MeshTable<VertexArgs> t)
 constexpr unsigned kLargeWaves = 8192;           // persistent wavefronts of the large-face pass
 constexpr unsigned kLargeItems = 8192;          // face parts that a short queue is split into
 constexpr int kLargePart = 512;                   // box pixels below which a large face is not split further
-// (view, face) items up to which the depth pass gives 16, or 4, lanes to a face instead of one.
+// (view, face) items up to which the depth pass gives 16, 8 or 2 lanes to a face instead of one.
 // A wavefront's time is a serial chain over its faces' lines and candidates, so with fewer than
 // about 4096 wavefronts the chain, not the chip, is the kernel's time: 20,480 items (4 x 256^2
-// sphere) took 126 us with one lane and 15 us with 16 lanes to a face; 245,760 items
-// (12 views of 517 x 389) 131 against 87 us with 4.  Above the line the per-face setup that the
-// lanes of a face repeat costs more than it gains (96,000 items with 16 lanes: forward + backward
-// 181 against 171 us with 4).  The meshes of a multi-mesh run fill the chip together, so their
-// items count together (8 uneven meshes: 2.10 ms when each mesh chose by its own, 1.86 ms).
-constexpr int64_t kRasterItems16 = 65536, kRasterItems4 = 262144;
+// sphere) took 126 us with one lane and 15 us with 16 lanes to a face; 245,760 items (12 views of
+// 517 x 389) forward alone 172 us with one lane, 146, 134 and 127 with 2, 4 and 8.  Further up the
+// lanes of a face still pay by the smaller staging area (one lane to a face holds 64 staged faces
+// and 6 wavefronts per SIMD, two lanes 8): 800,000 items forward + backward 647 us with one lane,
+// 631, 629 and 655 with 2, 4 and 8; then the setup that they repeat outweighs it (3.2 M items 1468,
+// 1475, 1531 us; 4.5 M items 1744, 1769, 1838 us).  The meshes of a multi-mesh run fill the chip
+// together, so their items count together (8 uneven meshes, choosing each by its own 2.10 ms,
+// together 1.56 with one lane, 1.54, 1.56 and 1.63 with 2, 4 and 8).
+constexpr int64_t kRasterItems16 = 65536, kRasterItems8 = 262144, kRasterItems2 = 2097152;
 
 struct RasterFace {
   int f, i0, i1, i2;
@@ -208,28 +211,34 @@ __device__ __forceinline__ RasterFace load_face(const int32_t* __restrict__ face
   return r;
 }
 
-// Per-face constants of the exact test, staged in LDS for the candidate pass: 64 bytes, so
-// that 64 staged faces and the candidate list take 5 KB and eight wavefronts fit per SIMD.
-// N.N is recomputed per candidate; the face id, view and box stay in registers (StageOwner).
-// Packed as four 16-byte words: (v0, v1.x), (v1.yz, v2.xy), (v2.z, N), (v0.N, z0, z1, z2), with
-// v0..v2 and N the scaled vertices and face normal of the ray/triangle test (TriSetup) and z0..z2
-// the projected depths.
-struct alignas(16) FaceStage {
-  float4 q[4];
+// Per-face constants of the exact test, staged in LDS for the candidate pass: the scaled vertices
+// and face normal of the ray/triangle test (TriSetup), v0.N - o.N for the face's view, the face id,
+// and the binary64 reciprocals of N.N and of the projected depths, which take a 14-cycle product
+// for each of the test's five divisions by them in the place of a 45-cycle division (quot).
+struct alignas(8) FaceStage {
+  float v[12];
+  float num;
+  int f;
+  double rden;
+  DepthRecip rz;
 };
+static_assert(sizeof(FaceStage) == 88, "staged face");
 
-__device__ __forceinline__ void stage_face(FaceStage* dst, const TriSetup& t, float z0, float z1, float z2) {
-  dst->q[0] = make_float4(t.v0.x, t.v0.y, t.v0.z, t.v1.x);
-  dst->q[1] = make_float4(t.v1.y, t.v1.z, t.v2.x, t.v2.y);
-  dst->q[2] = make_float4(t.v2.z, t.N.x, t.N.y, t.N.z);
-  dst->q[3] = make_float4(t.dv0N, z0, z1, z2);
+__device__ __forceinline__ void stage_face(FaceStage* dst, const TriSetup& t, V3 os, int f, float z0, float z1, float z2) {
+  const float v[12] = {t.v0.x, t.v0.y, t.v0.z, t.v1.x, t.v1.y, t.v1.z, t.v2.x, t.v2.y, t.v2.z, t.N.x, t.N.y, t.N.z};
+#pragma unroll
+  for (int k = 0; k < 12; ++k) dst->v[k] = v[k];
+  dst->num = t.dv0N - dot(os, t.N);
+  dst->f = f;
+  dst->rden = t.rden;
+  dst->rz = depth_recip(z0, z1, z2);
 }
 
 // Registers of the face a lane staged (its staging slot is that lane), read by the lanes that
 // test its candidates with a cross-lane permute (G lanes hold a face: the first is slot * G).
 // The large-face pass holds its one face in every lane.
 struct StageOwner {
-  int f, bc, x0, y0, bw;
+  int bc, x0, y0, bw;
 };
 
 // Candidate list of one wavefront: 32-bit words naming a staged face (its slot) and a pixel.
@@ -277,22 +286,24 @@ __device__ __forceinline__ void flush_candidates(const FaceStage* st, const Stag
       u = x0 + (int)(p - dy * w);
       v = y0 + (int)dy;
     }
-    const int f = __shfl(own.f, slot * G, 64);
     const int bc = one_view ? bc0 : __shfl(own.bc, slot * G, 64);
     if (!valid) continue;
-    const float4 q0 = st[slot].q[0], q1 = st[slot].q[1], q2 = st[slot].q[2], q3 = st[slot].q[3];
+    const FaceStage& fs = st[slot];
     const Camera& cam = cams[bc];
     const V3 d = pixel_ray(cam, u + 0.5f, v + 0.5f);
     TriSetup t;
-    t.v0 = v3(q0.x, q0.y, q0.z);
-    t.v1 = v3(q0.w, q1.x, q1.y);
-    t.v2 = v3(q1.z, q1.w, q2.x);
-    t.N = v3(q2.y, q2.z, q2.w);
-    t.dv0N = q3.x;
-    t.den = dot(t.N, t.N);      // as tri_setup forms it
-    const V3 abc = ray_barycentric(t, cam_origin_scaled(cam), d);
-    if (!inside(abc)) continue;
-    const uint64_t k = pack_key(depth_key(abc, q3.y, q3.z, q3.w), f);
+    t.v0 = v3(fs.v[0], fs.v[1], fs.v[2]);
+    t.v1 = v3(fs.v[3], fs.v[4], fs.v[5]);
+    t.v2 = v3(fs.v[6], fs.v[7], fs.v[8]);
+    t.N = v3(fs.v[9], fs.v[10], fs.v[11]);
+    t.den = dot(t.N, t.N);      // as tri_setup forms it; only a subnormal quotient divides by it
+    t.rden = fs.rden;
+    V3 abc;
+    // a and b of a hit are not negative, so that of inside()'s six bounds these three are left
+    if (!ray_hit(t, fs.num, cam_origin_scaled(cam), d, abc) || !(abc.x <= 1.001f) || !(abc.y <= 1.001f) ||
+        !(abc.z >= -0.001f))
+      continue;
+    const uint64_t k = pack_key(depth_key(abc, fs.rz), fs.f);
     atomicMin(keys + ((size_t)bc * H + v) * W + u, (unsigned long long)k);
     // screen-tile depth pass: the tile kernel merges this tile's visibility keys
     if (marks.dirty) marks.dirty[((size_t)bc * marks.tiles_y + (v >> marks.sy)) * marks.tiles_x + (u >> marks.sx)] = 1u;
@@ -387,9 +398,12 @@ __device__ __forceinline__ void append_spans(unsigned* cand, int& count, int rem
 // The G lanes of a face take its lines in turn.  On every step each lane finds the span of its
 // line, a wave sum of the span lengths gives each lane its place in the candidate list, and the
 // lanes write their spans there; a full list (always a multiple of 64) is tested and emptied.
-// Bound by VALU issue.  The spans replace an edge test of every box pixel, one pixel of 64 boxes
-// per step with 13.75 of the 64 lanes passing on average at 100k triangles over 8 x 1024^2 views:
-// 0.249 -> 0.153 ms there, 0.434 -> 0.330 ms at 200k triangles over 16 x 1024^2.
+// The spans replace an edge test of every box pixel, one pixel of 64 boxes per step with 13.75 of
+// the 64 lanes passing on average at 100k triangles over 8 x 1024^2 views: 249 -> 153 us there.
+// What bounds it now, there, is the memory side's rate of atomic requests: 2.59 M in 137 us, 19 G/s
+// of the 21 G/s that scattered atomics reach (the large-face pass the same, 0.72 M in 38 us), with
+// VALU issue at 60% (51 M instructions).  Reading a pixel's key before the exact test, to skip the
+// atomic where the face cannot win, adds a memory-side request for each it saves: 165 us.
 template <int G>
 __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
   constexpr int kFaces = 64 / G;
@@ -422,7 +436,8 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
         to_queue = sub == 0;
       } else {
         small = true;
-        if (sub == 0) stage_face(&st[slot], tris[(size_t)(bc / C) * F + f], r.p0.z, r.p1.z, r.p2.z);
+        if (sub == 0)
+          stage_face(&st[slot], tris[(size_t)(bc / C) * F + f], cam_origin_scaled(cams[bc]), f, r.p0.z, r.p1.z, r.p2.z);
         et = edge_test(r.p0, r.p1, r.p2);
         fx0 = r.bx.x0;
         fy0 = r.bx.y0;
@@ -444,7 +459,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
   if (!__ballot(small)) return;
   const int bc0 = __builtin_amdgcn_readfirstlane(bc);
   const bool one_view = __ballot(bc != bc0 && in_range) == 0;
-  const StageOwner own{f, bc, fx0, fy0, bw};
+  const StageOwner own{bc, fx0, fy0, bw};
   __syncthreads();
   int count = 0;
   const bool packed = cand_packed(W, H);
@@ -507,8 +522,9 @@ __device__ __forceinline__ void raster_large_face(const TriSetup* __restrict__ t
   bl.start(edge_test(r.p0, r.p1, r.p2), r.bx.x0, r.bx.y0, bw, bh);
   const int lane = threadIdx.x & 63;
   wave_sync();
-  if (lane == 0) stage_face(&st[0], tris[(size_t)(bc / C) * F + f], r.p0.z, r.p1.z, r.p2.z);
-  const StageOwner own{f, bc, r.bx.x0, r.bx.y0, bw};
+  if (lane == 0)
+    stage_face(&st[0], tris[(size_t)(bc / C) * F + f], cam_origin_scaled(cams[bc]), f, r.p0.z, r.p1.z, r.p2.z);
+  const StageOwner own{bc, r.bx.x0, r.bx.y0, bw};
   wave_sync();
   const bool packed = cand_packed(W, H);
   const unsigned step = cand_word(packed, true, 0, bl.columns ? 0 : 1, bl.columns ? 1 : 0, bl.columns ? 0 : 1,
@@ -751,12 +767,12 @@ hipError_t launch_raster_large_multi(const RasterMesh* meshes, unsigned int* cou
 
 static void launch_raster(const ForwardPlan& p, const RasterArgs& ra, hipStream_t s) {
   const int64_t items = (int64_t)ra.B * ra.C * ra.F;
-  if (p.raster_items <= kRasterItems16)
-    hipLaunchKernelGGL(k_raster<16>, dim3(blocks_for(items, 4)), dim3(64), 0, s, ra);
-  else if (p.raster_items <= kRasterItems4)
-    hipLaunchKernelGGL(k_raster<4>, dim3(blocks_for(items, 16)), dim3(64), 0, s, ra);
-  else
-    hipLaunchKernelGGL(k_raster<1>, dim3(blocks_for(items, 64)), dim3(64), 0, s, ra);
+  const int g = p.raster_items <= kRasterItems16 ? 16 : p.raster_items <= kRasterItems8 ? 8 : p.raster_items <= kRasterItems2 ? 2 : 1;
+  const dim3 grid(blocks_for(items, 64 / g));
+  if (g == 16) hipLaunchKernelGGL(k_raster<16>, grid, dim3(64), 0, s, ra);
+  else if (g == 8) hipLaunchKernelGGL(k_raster<8>, grid, dim3(64), 0, s, ra);
+  else if (g == 2) hipLaunchKernelGGL(k_raster<2>, grid, dim3(64), 0, s, ra);
+  else hipLaunchKernelGGL(k_raster<1>, grid, dim3(64), 0, s, ra);
 }
 
 hipError_t launch_forward_raster(const ForwardPlan& p, hipStream_t s) {

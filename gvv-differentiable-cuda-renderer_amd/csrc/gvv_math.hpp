@@ -28,15 +28,77 @@ GVV_HD V3 operator*(float s, V3 a) { return v3(s * a.x, s * a.y, s * a.z); }
 GVV_HD V3 operator/(V3 a, float s) { return v3(a.x / s, a.y / s, a.z / s); }
 GVV_HD float dot(V3 a, V3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 GVV_HD V3 cross(V3 a, V3 b) { return v3(a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x); }
-GVV_HD float length(V3 a) { return sqrtf(dot(a, a)); }
-GVV_HD V3 normalize(V3 a) { float inv = 1.0f / sqrtf(dot(a, a)); return a * inv; }
+
+// Correctly rounded reciprocals, square roots and quotients, bit for bit what the IEEE operations
+// give, in fewer instructions than the compiler's sequences, which scale for the whole binary32
+// range first: in cycles of one SIMD for 64 lanes, 45 for a division, 54 for a square root, 98 for
+// 1 / sqrt, against 4.8 for an FMA.  On the host they are the IEEE operations themselves.
+//   rcp_rn       one Newton step on the 1-ulp hardware reciprocal (17 cycles).  Every binary32 x
+//                with 2^-100 <= |x| < 2^100 was compared with 1 / x on the device; others divide.
+//   sqrt_rn      one correction of x rsq(x) (27 cycles), compared likewise for every x in that
+//                range; others take sqrtf.
+//   quot         a / b from a binary64 reciprocal r of b (recip64, within 2^-52 of 1 / b): one
+//                binary64 product, rounded to binary32 (14 cycles).  The quotient of two 24-bit
+//                significands is at least 2^-49 (relative) from the midpoint of two binary32
+//                numbers and the product is within 2^-51 of it, so the rounding is that of the exact
+//                quotient, for every normal result; a subnormal one divides.
+constexpr float kRnMin = 0x1p-100f, kRnMax = 0x1p100f;
+GVV_HD float rcp_rn(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (fabsf(x) >= kRnMin && fabsf(x) < kRnMax) {
+    const float y = __builtin_amdgcn_rcpf(x);
+    return fmaf(fmaf(-x, y, 1.f), y, y);
+  }
+#endif
+  return 1.0f / x;
+}
+GVV_HD float sqrt_rn(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (x >= kRnMin && x < kRnMax) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s = x * y;
+    return fmaf(fmaf(-s, s, x), 0.5f * y, s);
+  }
+#endif
+  return sqrtf(x);
+}
+GVV_HD double recip64(float b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (fabsf(b) >= kRnMin && fabsf(b) < kRnMax) {
+    const double x = b;
+    double y = __builtin_amdgcn_rcpf(b);      // within 2^-23; 2^-46 and 2^-52 after the steps
+    y = fma(fma(-x, y, 1.0), y, y);
+    return fma(fma(-x, y, 1.0), y, y);
+  }
+#endif
+  return 1.0 / (double)b;
+}
+GVV_HD float quot(float a, float b, double r) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float q = (float)((double)a * r);
+  return fabsf(q) >= 0x1p-126f || a == 0.f ? q : a / b;
+#else
+  (void)r;
+  return a / b;
+#endif
+}
+
+GVV_HD float length(V3 a) { return sqrt_rn(dot(a, a)); }
+GVV_HD V3 normalize(V3 a) { float inv = rcp_rn(sqrt_rn(dot(a, a))); return a * inv; }
 GVV_HD V3 ld3(const float* p) { return v3(p[0], p[1], p[2]); }
 
+// Truncation to int32, saturating, NaN -> 0: what the device's conversion instruction does.
 GVV_HD int32_t sat_i32(float z) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  int32_t i;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(z));
+  return i;
+#else
   if (!(z == z)) return 0;
   if (z >= 2147483648.0f) return INT32_MAX;
   if (z <= -2147483648.0f) return INT32_MIN;
   return (int32_t)z;
+#endif
 }
 
 // Visibility key: ascending in (depth key, face id); all-ones marks an empty pixel.
@@ -165,7 +227,7 @@ struct alignas(16) TriSetup {
   V3 N;            // cross(v1 - v0, v2 - v0)
   float dv0N;      // dot(v0, N)
   float den;       // dot(N, N)
-  float pad[2];
+  double rden;     // its reciprocal (recip64), for the quotients by den
 };
 
 GVV_HD TriSetup tri_setup(V3 v0, V3 v1, V3 v2) {
@@ -174,26 +236,29 @@ GVV_HD TriSetup tri_setup(V3 v0, V3 v1, V3 v2) {
   t.N = cross(t.v1 - t.v0, t.v2 - t.v0);
   t.dv0N = dot(t.v0, t.N);
   t.den = dot(t.N, t.N);
-  t.pad[0] = t.pad[1] = 0.f;
+  t.rden = recip64(t.den);
   return t;
 }
 
-// Barycentrics (a -> v0, b -> v1, c -> v2) of the ray hit, or (-1,-1,-1) on a miss.
-// o_s is the ray origin already divided by 1000.
-GVV_HD V3 ray_barycentric(const TriSetup& t, V3 o_s, V3 d) {
-  const V3 miss = v3(-1.f, -1.f, -1.f);
-  float ndr = dot(d, t.N);
-  if (fabsf(ndr) < 0.0000001f) return miss;
-  float tt = (t.dv0N - dot(o_s, t.N)) / ndr;
-  if (tt < 0) return miss;
-  V3 P = o_s + tt * d;
-  if (dot(t.N, cross(t.v1 - t.v0, P - t.v0)) < 0) return miss;
+// Barycentrics (a -> v0, b -> v1, c -> v2) of the ray hit; false on a miss.  num: dot(v0, N) -
+// dot(o_s, N) with o_s the ray origin already divided by 1000.
+GVV_HD bool ray_hit(const TriSetup& t, float num, V3 o_s, V3 d, V3& abc) {
+  const float ndr = dot(d, t.N);
+  const float tt = num / ndr;
+  const V3 P = o_s + tt * d;
+  const float s = dot(t.N, cross(t.v1 - t.v0, P - t.v0));
   float a = dot(t.N, cross(t.v2 - t.v1, P - t.v1));
-  if (a < 0) return miss;
   float b = dot(t.N, cross(t.v0 - t.v2, P - t.v2));
-  if (b < 0) return miss;
-  a /= t.den; b /= t.den;
-  return v3(a, b, 1.f - a - b);
+  const bool miss = fabsf(ndr) < 0.0000001f || tt < 0 || s < 0 || a < 0 || b < 0;
+  a = quot(a, t.den, t.rden); b = quot(b, t.den, t.rden);
+  abc = v3(a, b, 1.f - a - b);
+  return !miss;
+}
+
+// The same with (-1,-1,-1) on a miss.
+GVV_HD V3 ray_barycentric(const TriSetup& t, V3 o_s, V3 d) {
+  V3 abc;
+  return ray_hit(t, t.dv0N - dot(o_s, t.N), o_s, d, abc) ? abc : v3(-1.f, -1.f, -1.f);
 }
 
 GVV_HD bool inside(V3 abc) {
@@ -201,16 +266,46 @@ GVV_HD bool inside(V3 abc) {
          (abc.x <= 1.001f) && (abc.y <= 1.001f) && (abc.z <= 1.001f);
 }
 
+// The integer depth key 10000 / (a / z0 + b / z1 + c / z2).
 GVV_HD int32_t depth_key(V3 abc, float z0, float z1, float z2) {
   float z = 1.f / (abc.x / z0 + abc.y / z1 + abc.z / z2);
   z *= 10000.f;
   return sat_i32(z);
 }
 
+// The same from the binary64 reciprocals of the depths, formed once per face and view, for the
+// barycentrics of an inside hit.  Depths (at least 1e-7 by the projection's clamp) below 2^60 give
+// quotients as quot() does; one that is subnormal comes from a barycentric below 2^-60, and the
+// sum with the other two, one of which is at least 2^-62, rounds it away whatever its own rounding.
+// Larger depths are kept as they are, marked by the sign of the first, and divide.
+struct DepthRecip {
+  double r0, r1, r2;
+};
+GVV_HD DepthRecip depth_recip(float z0, float z1, float z2) {
+  DepthRecip r;
+  if (z0 >= 0x1p60f || z1 >= 0x1p60f || z2 >= 0x1p60f) {
+    r.r0 = -(double)z0; r.r1 = z1; r.r2 = z2;
+  } else {
+    r.r0 = recip64(z0); r.r1 = recip64(z1); r.r2 = recip64(z2);
+  }
+  return r;
+}
+GVV_HD int32_t depth_key(V3 abc, DepthRecip r) {
+  if (r.r0 < 0.0) return depth_key(abc, (float)-r.r0, (float)r.r1, (float)r.r2);
+  const float s = (float)((double)abc.x * r.r0) + (float)((double)abc.y * r.r1) + (float)((double)abc.z * r.r2);
+  return sat_i32(rcp_rn(s) * 10000.f);
+}
+
+// a / l by component.
+GVV_HD V3 over(V3 a, float l) {
+  const double r = recip64(l);
+  return v3(quot(a.x, l, r), quot(a.y, l, r), quot(a.z, l, r));
+}
+
 // Interpolated, normalised vertex normal (before any flip).
 GVV_HD V3 pixel_normal(V3 n0, V3 n1, V3 n2, V3 abc) {
   V3 n = n0 * abc.x + n1 * abc.y + n2 * abc.z;
-  return n / length(n);
+  return over(n, length(n));
 }
 
 struct TexCoord { float U0, V0; int LU, LV; };

@@ -16,7 +16,7 @@ EXPORTS = ("gvv_last_error", "gvv_version", "gvv_create", "gvv_destroy", "gvv_fo
            "gvv_backward_noalloc",
            "gvv_profile_enable", "gvv_profile_report", "gvv_set_tuning", "gvv_get_tuning",
            "gvv_set_depth_pass", "gvv_get_depth_pass",
-           "gvv_calibrate_atomics",
+           "gvv_calibrate_atomics", "gvv_check_rounding",
            "gvv_conv_out_size", "gvv_conv_forward", "gvv_conv_backward_data", "gvv_conv_workspace_floats",
            "gvv_conv_backward_weight", "gvv_conv_prepare_weights", "gvv_conv_prepare_weights_layers",
            "gvv_pack_mosaic",
@@ -61,6 +61,8 @@ def load():
     L.gvv_profile_report.restype = i64
     L.gvv_calibrate_atomics.argtypes = [P, i64, i64, i32, P]
     L.gvv_calibrate_atomics.restype = ctypes.c_int
+    L.gvv_check_rounding.argtypes = [ctypes.c_uint64, ctypes.c_uint64, P, P]
+    L.gvv_check_rounding.restype = ctypes.c_int
     L.gvv_set_tuning.argtypes = [P, i32, i32]
     L.gvv_set_tuning.restype = ctypes.c_int
     L.gvv_get_tuning.argtypes = [P, ctypes.POINTER(i32), ctypes.POINTER(i32)]

@@ -135,6 +135,12 @@ int gvv_get_depth_pass(void* handle, int32_t* mode);
  * can time the GPU's float-atomic throughput.  Overwrites buf. */
 int gvv_calibrate_atomics(float* buf, int64_t n_floats, int64_t updates, int32_t scattered, void* stream);
 
+/* Self-check of the renderer's correctly rounded device arithmetic: for every binary32 bit pattern
+ * in [first, first + count), adds to mismatches[0..4] (device counters the caller cleared) where the
+ * reciprocal, the square root, quotients, the conversion to int32 and the depth key differ from the
+ * IEEE operations. */
+int gvv_check_rounding(uint64_t first, uint64_t count, uint64_t* mismatches, void* stream);
+
 /* Kernel timing (no counterpart in the reference, which has no timing code).  When enabled,
  * every kernel launch of this handle is bracketed by HIP events on its stream; enabling or
  * disabling clears the accumulated figures. */
