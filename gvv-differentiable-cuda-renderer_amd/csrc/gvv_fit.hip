@@ -9,9 +9,9 @@
 // under a rigid motion per subject, and the gradients of alpha and of (R, t).  The forward is
 // one thread per vertex and group of 4 subjects (the coefficients and motions are wave-uniform
 // scalar loads).  The backward sums over vertices:
-// each workgroup takes a chunk of vertices, stages the chunk of the basis and the subjects'
-// unrotated vertex gradients in LDS and forms every (subject, coefficient) partial dot
-// product of the chunk; a second launch adds the chunks' partials in a fixed order.
+// each workgroup takes a chunk of vertices, stages the subjects' unrotated vertex gradients in LDS
+// and forms every (subject, coefficient) partial dot product of the chunk with FP32 MFMAs, the
+// basis straight from memory; a second launch adds the chunks' partials in a fixed order.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -102,42 +102,60 @@ __global__ void __launch_bounds__(kThreads) k_masked_sq_grad(const float* __rest
 constexpr int kShapeSubjects = 16;     // subjects per backward workgroup (grid.y covers more)
 constexpr int kShapeMaxSubjects = 65535 * 4;   // the forward's grid.y limit at 4 subjects per thread
 constexpr int kShapeChunk = 64;        // vertices per backward workgroup
-constexpr int kShapeRow = 3 * kShapeChunk + 1;   // padded LDS row: lanes of one column differ in bank
+constexpr int kShapeRow = 3 * kShapeChunk + 4;   // padded LDS row: 16-byte reads of 16 rows spread over the banks
+constexpr int kShapeWaves = 4;         // waves of a backward workgroup, each with a quarter of the chunk
 constexpr int kShapeMaxBasis = 128;
 constexpr int kShapeRt = 12;           // R row-major (9) and t (3) per subject
 
 // v[b][i] = R_b (T_i + sum_k alpha[b][k] basis[k][3i..3i+2] - c) + c + t_b and xc[b][i] = the
 // unrotated, centred vertex (T_i + ... - c), kept for the backward.  Thread = (vertex, group of
-// kShapeFwdSubjects subjects b0 .. b0 + nb - 1): enough wavefronts to cover the basis reads'
-// latency, which one thread per vertex for all subjects leaves exposed.
+// kShapeFwdSubjects subjects b0 .. b0 + nb - 1).  Bound by the basis reads: the groups of the same
+// 64 vertices are the waves of one workgroup, so the basis comes from memory once for 16 subjects,
+// and kShapeUnroll rows of it are in flight per thread (16 subjects, 35,002 vertices, 80 rows:
+// 15 us; with a workgroup of its own per group and no more loads in flight than the compiler kept,
+// 42).
 constexpr int kShapeFwdSubjects = 4;
+constexpr int kShapeFwdGroups = 4;
+constexpr int kShapeUnroll = 8;
 
-__global__ void __launch_bounds__(64) k_shape_forward(const float* __restrict__ alpha, const float* __restrict__ rt,
-                                                      const float* __restrict__ templ, const float* __restrict__ basis,
-                                                      const float* __restrict__ centre, int B, int N, int K,
-                                                      float* __restrict__ v, float* __restrict__ xc) {
-  const int i = blockIdx.x * 64 + threadIdx.x;
-  const int b0 = blockIdx.y * kShapeFwdSubjects;
+__global__ void __launch_bounds__(64 * kShapeFwdGroups) k_shape_forward(
+    const float* __restrict__ alpha, const float* __restrict__ rt, const float* __restrict__ templ,
+    const float* __restrict__ basis, const float* __restrict__ centre, int B, int N, int K, float* __restrict__ v,
+    float* __restrict__ xc) {
+  const int i = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int group = blockIdx.y * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b0 = group * kShapeFwdSubjects;
   const int nb = B - b0 < kShapeFwdSubjects ? B - b0 : kShapeFwdSubjects;
-  if (i >= N) return;
+  if (i >= N || nb <= 0) return;
   float acc[kShapeFwdSubjects][3];
 #pragma unroll
   for (int s = 0; s < kShapeFwdSubjects; ++s) acc[s][0] = acc[s][1] = acc[s][2] = 0.f;
   const size_t n3 = (size_t)3 * N;
   const float* bi = basis + 3 * (size_t)i;
-#pragma unroll 4
-  for (int k = 0; k < K; ++k) {
-    const float e0 = bi[k * n3], e1 = bi[k * n3 + 1], e2 = bi[k * n3 + 2];
+  const float* al[kShapeFwdSubjects];          // subjects past the end repeat the last one
+#pragma unroll
+  for (int s = 0; s < kShapeFwdSubjects; ++s) al[s] = alpha + (size_t)min(b0 + s, B - 1) * K;
+  auto add = [&](int k, float e0, float e1, float e2) {
 #pragma unroll
     for (int s = 0; s < kShapeFwdSubjects; ++s) {
-      if (s < nb) {
-        const float a = alpha[(size_t)(b0 + s) * K + k];
-        acc[s][0] += a * e0;
-        acc[s][1] += a * e1;
-        acc[s][2] += a * e2;
-      }
+      const float a = al[s][k];
+      acc[s][0] += a * e0;
+      acc[s][1] += a * e1;
+      acc[s][2] += a * e2;
     }
+  };
+  int k0 = 0;
+  for (; k0 + kShapeUnroll <= K; k0 += kShapeUnroll) {
+    float e[kShapeUnroll][3];
+#pragma unroll
+    for (int u = 0; u < kShapeUnroll; ++u)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) e[u][c] = bi[(size_t)(k0 + u) * n3 + c];
+    __builtin_amdgcn_sched_barrier(0);       // every load of the block before the first use
+#pragma unroll
+    for (int u = 0; u < kShapeUnroll; ++u) add(k0 + u, e[u][0], e[u][1], e[u][2]);
   }
+  for (; k0 < K; ++k0) add(k0, bi[k0 * n3], bi[k0 * n3 + 1], bi[k0 * n3 + 2]);
   const float c0 = centre[0], c1 = centre[1], c2 = centre[2];
   const float t0 = templ[3 * (size_t)i], t1 = templ[3 * (size_t)i + 1], t2 = templ[3 * (size_t)i + 2];
 #pragma unroll
@@ -156,16 +174,23 @@ __global__ void __launch_bounds__(64) k_shape_forward(const float* __restrict__ 
 
 // Workgroup (chunk j, subject group): partial[j][b][0..K) = sum over the chunk's vertices of
 // (R_b^T g_v[b][i]) . basis[k][3i..3i+2], and partial[j][b][K..K+12) the chunk's sums of
-// g_v[b][i] (x) xc[b][i] (9, row-major) and of g_v[b][i] (3).  Dynamic LDS: (K + 16) padded
-// rows of the chunk (basis rows, then the subjects' unrotated gradients).
-__global__ void __launch_bounds__(256) k_shape_backward_partial(const float* __restrict__ g_v,
+// g_v[b][i] (x) xc[b][i] (9, row-major) and of g_v[b][i] (3).
+// The dot products are a [16 subjects] x [K] product over the chunk's 192 coordinates, on
+// v_mfma_f32_16x16x4_f32: lane l holds subject l % 16 (A) and basis row l % 16 (B) at coordinate
+// l / 16 of a step, and four steps take one 16-byte load of each (coordinates 4 (l / 16) + step:
+// the sum's order is free).  The waves take 48 coordinates each and add their sums through LDS.
+// Bound by the basis reads (33.6 MB at 35,002 vertices and 80 rows: 16 us).  Staging the basis in LDS
+// with two LDS reads per product took 59 us.
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+
+__global__ void __launch_bounds__(64 * kShapeWaves) k_shape_backward_partial(const float* __restrict__ g_v,
                                                                 const float* __restrict__ xc,
                                                                 const float* __restrict__ rt,
                                                                 const float* __restrict__ basis, int B, int N, int K,
                                                                 float* __restrict__ partial) {
-  extern __shared__ float s_rows[];
-  float* s_basis = s_rows;                       // [K][kShapeRow]
-  float* s_g = s_rows + (size_t)K * kShapeRow;   // [16][kShapeRow]
+  constexpr int kTiles = kShapeMaxBasis / 16;
+  __shared__ __attribute__((aligned(16))) float s_g[kShapeSubjects * kShapeRow];
+  __shared__ float s_sum[kShapeWaves - 1][kTiles * 4][64];
   const int tid = threadIdx.x;
   const int j = blockIdx.x;
   const int i0 = j * kShapeChunk;
@@ -174,29 +199,39 @@ __global__ void __launch_bounds__(256) k_shape_backward_partial(const float* __r
   const int nb = B - b0 < kShapeSubjects ? B - b0 : kShapeSubjects;
   const int stride = K + kShapeRt;
   const size_t n3 = (size_t)3 * N;
-  // the chunk of every basis row (coalesced along the row), four loads in flight per thread
-  const int total = K * 3 * kShapeChunk;
-  for (int q0 = tid; q0 < total; q0 += 4 * 256) {
-    float e[4];
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), row = lane & 15, kg = lane >> 4;
+  const int tiles = (K + 15) / 16;
+  // this wave's quarter of the chunk: 3 groups of 16 coordinates, 4 of them per lane
+  constexpr int kGroups = 3 * kShapeChunk / kShapeWaves / 16;
+  auto load = [&](int tile, int grp) {
+    const int k = tile * 16 + row, c = (wave * kGroups + grp) * 16 + 4 * kg;
+    f32x4 e = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (k < K) {
+      const float* src = basis + k * n3 + 3 * (size_t)i0 + c;
+      if (c + 3 < 3 * nv) {
+        __builtin_memcpy(&e, src, 16);
+      } else {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int q = q0 + u * 256;
-      const int k = q / (3 * kShapeChunk), c = q - k * 3 * kShapeChunk;
-      e[u] = q < total && c < 3 * nv ? basis[k * n3 + 3 * (size_t)i0 + c] : 0.f;
+        for (int u = 0; u < 4; ++u)
+          if (c + u < 3 * nv) e[u] = src[u];
+      }
     }
+    return e;
+  };
+  f32x4 eb[2][kGroups];          // the basis of this tile and the next
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int q = q0 + u * 256;
-      const int k = q / (3 * kShapeChunk), c = q - k * 3 * kShapeChunk;
-      if (q < total) s_basis[k * kShapeRow + c] = e[u];
-    }
-  }
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int q = 0; q < kGroups; ++q)
+      if (t < tiles) eb[t][q] = load(t, q);
   // 16 lanes per subject, 4 vertices each: unrotated gradients into LDS, motion sums in registers
   {
     const int s = tid >> 4, l = tid & 15;
     float acc[kShapeRt];
 #pragma unroll
     for (int q = 0; q < kShapeRt; ++q) acc[q] = 0.f;
+    for (int vv = l; s >= nb && vv < kShapeChunk; vv += 16)
+      s_g[s * kShapeRow + 3 * vv] = s_g[s * kShapeRow + 3 * vv + 1] = s_g[s * kShapeRow + 3 * vv + 2] = 0.f;
     if (s < nb) {
       const float* m = rt + (size_t)(b0 + s) * kShapeRt;
       for (int vv = l; vv < kShapeChunk; vv += 16) {
@@ -230,14 +265,48 @@ __global__ void __launch_bounds__(256) k_shape_backward_partial(const float* __r
     }
   }
   __syncthreads();
-  // every (subject, coefficient) dot product over the chunk
-  for (int o = tid; o < nb * K; o += 256) {
-    const int s = o / K, k = o - s * K;
-    const float* gr = s_g + s * kShapeRow;
-    const float* br = s_basis + k * kShapeRow;
-    float a = 0.f;
-    for (int c = 0; c < 3 * nv; ++c) a += gr[c] * br[c];
-    partial[((size_t)j * B + b0 + s) * stride + k] = a;
+  // every (subject, coefficient) dot product over this wave's coordinates, 16 coefficients at a time
+  f32x4 ga[kGroups];
+#pragma unroll
+  for (int q = 0; q < kGroups; ++q)
+    ga[q] = *reinterpret_cast<const f32x4*>(s_g + row * kShapeRow + (wave * kGroups + q) * 16 + 4 * kg);
+  f32x4 acc[kTiles];
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) {
+    acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (t < tiles) {
+#pragma unroll
+      for (int q = 0; q < kGroups; ++q)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ga[q][u], eb[t & 1][q][u], acc[t], 0, 0, 0);
+#pragma unroll
+      for (int q = 0; q < kGroups; ++q)
+        if (t + 2 < tiles) eb[t & 1][q] = load(t + 2, q);
+    }
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+      if (t < tiles)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s_sum[wave - 1][4 * t + u][lane] = acc[t][u];
+  }
+  __syncthreads();
+  if (wave == 0) {
+    // lane: coefficient 16 t + row of subjects 4 kg .. 4 kg + 3
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      const int k = 16 * t + row;
+      if (t < tiles && k < K) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          float a = acc[t][u];
+#pragma unroll
+          for (int w = 0; w < kShapeWaves - 1; ++w) a += s_sum[w][4 * t + u][lane];
+          if (4 * kg + u < nb) partial[((size_t)j * B + b0 + 4 * kg + u) * stride + k] = a;
+        }
+      }
+    }
   }
 }
 
@@ -414,8 +483,10 @@ extern "C" int gvv_shape_forward(int32_t B, int32_t N, int32_t K, const float* a
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(k_pose_motion, dim3((unsigned)((B + 63) / 64)), dim3(64), 0, s, pose, tscale, B, rt);
   if (!check_launch("shape forward")) return 1;
-  const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((B + kShapeFwdSubjects - 1) / kShapeFwdSubjects));
-  hipLaunchKernelGGL(k_shape_forward, grid, dim3(64), 0, s, alpha, rt, templ, basis, centre, B, N, K, v, xc);
+  const int groups = (B + kShapeFwdSubjects - 1) / kShapeFwdSubjects;
+  const int per = groups < kShapeFwdGroups ? groups : kShapeFwdGroups;      // waves of a workgroup
+  const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((groups + per - 1) / per));
+  hipLaunchKernelGGL(k_shape_forward, grid, dim3(64 * per), 0, s, alpha, rt, templ, basis, centre, B, N, K, v, xc);
   return check_launch("shape forward") ? 0 : 1;
 }
 
@@ -428,14 +499,9 @@ extern "C" int gvv_shape_backward(int32_t B, int32_t N, int32_t K, const float* 
     return gvv::set_last_error("shape backward: null pointer");
   const int chunks = (N + kShapeChunk - 1) / kShapeChunk;
   const int stride = K + kShapeRt;
-  const size_t lds = (size_t)(K + kShapeSubjects) * kShapeRow * sizeof(float);   // <= 111 KB at K = 128
-  // dynamic LDS above 64 KB needs the attribute (set on the current device)
-  const hipError_t e = hipFuncSetAttribute((const void*)k_shape_backward_partial,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return gvv::set_last_error(std::string("shape backward: ") + hipGetErrorString(e));
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid((unsigned)chunks, (unsigned)((B + kShapeSubjects - 1) / kShapeSubjects));
-  hipLaunchKernelGGL(k_shape_backward_partial, grid, dim3(256), lds, s, g_v, xc, rt, basis, B, N, K, work);
+  hipLaunchKernelGGL(k_shape_backward_partial, grid, dim3(64 * kShapeWaves), 0, s, g_v, xc, rt, basis, B, N, K, work);
   if (!check_launch("shape backward")) return 1;
   float* sums = work + (size_t)chunks * B * stride;
   const int64_t outs = (int64_t)B * stride;
