@@ -9,7 +9,6 @@ libgvv_amd.so on the caller's current HIP stream.
 from __future__ import annotations
 
 import ctypes
-import hashlib
 import threading
 
 import numpy as np
@@ -22,11 +21,14 @@ SHADING_MODES = {"shaded": 0, "shadeless": 1}
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _stream_ptr(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current HIP stream of a device (what torch.cuda.current_stream(device).cuda_stream says,
+    without making a Stream object: 0.1 us instead of 1.9)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 class Rasterizer:
@@ -249,8 +251,31 @@ _cache_lock = threading.Lock()
 _CACHE_MAX = 32
 
 
-def _digest(a):
-    return hashlib.blake2b(np.ascontiguousarray(a).tobytes(), digest_size=16).hexdigest()
+_memcmp = ctypes.CDLL(None).memcmp
+_memcmp.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t]
+_memcmp.restype = ctypes.c_int
+
+
+class _Content:
+    """An array as part of a cache key: equal when every byte is.  Its hash is that of a sample of 64
+    values, so that a lookup costs one comparison (12,000 values: 2 us) in the place of a digest of
+    everything (33 us).  A key that stays in a cache owns its values (`own`)."""
+    __slots__ = ("a", "h")
+
+    def __init__(self, a):
+        self.a = np.ascontiguousarray(a)
+        self.h = hash((self.a.size, self.a[::max(1, self.a.size // 64)].tobytes()))
+
+    def own(self):
+        self.a = self.a.copy()
+
+    def __hash__(self):
+        return self.h
+
+    def __eq__(self, other):
+        return (isinstance(other, _Content) and self.h == other.h and self.a.nbytes == other.a.nbytes and
+                self.a.dtype == other.a.dtype and
+                _memcmp(self.a.ctypes.data, other.a.ctypes.data, self.a.nbytes) == 0)
 
 
 def cache_key(faces, texture_coordinates, number_of_vertices, number_of_cameras, render_resolution_u,
@@ -262,7 +287,7 @@ def cache_key(faces, texture_coordinates, number_of_vertices, number_of_cameras,
     the host-side lock of a handle cannot order on the GPU -- gets two handles."""
     faces = np.asarray(faces, dtype=np.int32).reshape(-1)
     tc = np.asarray(texture_coordinates, dtype=np.float32).reshape(-1)
-    return (_digest(faces), _digest(tc), int(number_of_vertices), int(number_of_cameras), int(render_resolution_u),
+    return (_Content(faces), _Content(tc), int(number_of_vertices), int(number_of_cameras), int(render_resolution_u),
             int(render_resolution_v), albedo_mode, shading_mode, int(image_filter_size), int(texture_filter_size),
             bool(compute_normal_map), int(device_index), int(stream_id))
 
@@ -274,7 +299,7 @@ def get_rasterizer(faces, texture_coordinates, number_of_vertices, number_of_cam
     dev = torch.cuda.current_device()
     key = cache_key(faces, texture_coordinates, number_of_vertices, number_of_cameras, render_resolution_u,
                     render_resolution_v, albedo_mode, shading_mode, image_filter_size, texture_filter_size,
-                    compute_normal_map, dev, torch.cuda.current_stream(dev).cuda_stream)
+                    compute_normal_map, dev, torch._C._cuda_getCurrentRawStream(dev))
     with _cache_lock:
         r = _cache.get(key)
         if r is None:
@@ -283,6 +308,8 @@ def get_rasterizer(faces, texture_coordinates, number_of_vertices, number_of_cam
                            compute_normal_map)
             if len(_cache) >= _CACHE_MAX:
                 _cache.pop(next(iter(_cache)))
+            for part in key[:2]:
+                part.own()       # the caller's arrays may change after this call
             _cache[key] = r
         return r
 
