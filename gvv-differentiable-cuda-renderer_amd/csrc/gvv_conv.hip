@@ -651,7 +651,9 @@ int launch(ConvArgs a, hipStream_t s, const char* what) {
 // tile reads its operands fewer times.  With 1024 tiles and more, one wave per tile fills the chip
 // and passes no accumulators (backward data of the 64-channel layer at 16 images: 29 us against 38
 // with four waves, of the 128-channel layer 24 against 28); with fewer, the stretches of the
-// reduction are loaded side by side (the 4096-deep head: 15 us, one wave 75).  Tiles of 32 x 128 and
+// reduction are loaded side by side, all at once where the waves' registers hold them (the 4096-deep
+// head of one image: 13 us with 16 waves, 21 with 8 and two rounds of loads, 75 with one wave; the
+// 2304-deep layer 9.4 us with 8 waves, 11.8 with 16, whose accumulators travel twice as far).  Tiles of 32 x 128 and
 // 64 x 128 were no faster (30 and 30 us for those two).
 template <bool FWD>
 int launch_conv(const ConvArgs& a, hipStream_t s, const char* what) {
@@ -666,7 +668,8 @@ int launch_conv(const ConvArgs& a, hipStream_t s, const char* what) {
   if (P > 32 && tiles(64, 64) >= 1024) return launch<FWD, 4, 4, 1, 2>(a, s, what);
   if (P > 32 && tiles(64, 64) >= 256) return launch<FWD, 4, 4, 4, 3>(a, s, what);
   if (P > 16 && tiles(32, 32) >= 256) return launch<FWD, 2, 2, 8, 5>(a, s, what);
-  return steps < 16 ? launch<FWD, 1, 1, 4, 4>(a, s, what) : launch<FWD, 1, 1, 16, 8>(a, s, what);
+  if (steps < 16) return launch<FWD, 1, 1, 4, 4>(a, s, what);
+  return steps <= 80 ? launch<FWD, 1, 1, 8, 10>(a, s, what) : launch<FWD, 1, 1, 16, 8>(a, s, what);
 }
 
 // Split of the weight-gradient reduction over workgroups: enough workgroups for the chip
