@@ -8,8 +8,8 @@
 //                  model-to-data and normal terms, from the face's ray/triangle and Jacobian
 //                  constants (FaceGrad, one 128-byte line per face, written by the setup
 //                  launch).  Per-face terms are summed in LDS slots (one per distinct face of
-//                  the tile) before lane-parallel global atomics flush them to the face's three
-//                  vertices; in the shaded modes a vertex's position and normal terms share one
+//                  the tile, a few faces' slots also over the corners of a vertex) before
+//                  lane-parallel global atomics flush them to the faces' vertices; in the shaded modes a vertex's position and normal terms share one
 //                  24-byte row of a scratch buffer, so that they cost one atomic request rather
 //                  than two.  SH terms accumulate in registers over the tile and are reduced
 //                  once per tile (a transposed DPP sum) into a partial buffer.
@@ -302,10 +302,10 @@ __device__ __forceinline__ void pixel_terms(const BackwardArgs& a, const Camera&
 // Per-face terms: every distinct face of the tile gets a slot in LDS (every lane finds or
 // inserts its face in an LDS hash table at once, and the inserting lanes number the new slots
 // in lane order); lanes add their terms into their face's slot with LDS atomics, and the
-// slots are flushed with lane-parallel global atomics (one per face, vertex and component).
+// slots are flushed with lane-parallel global atomics (one per face, vertex and component; with few
+// faces one per vertex and component).
 // SH terms accumulate in registers over the tile and are reduced once into the tile's
 // partial slots.
-constexpr int kFaceSlots = 96;
 constexpr int kHashCap = 128;
 
 // COL_GRAD: the vertex-colour gradient is formed (vertexColor mode with a g_col output).
@@ -318,8 +318,16 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
   constexpr int G_POS = 0, G_VN = NEED_POS ? 9 : 0, G_COL = G_VN + (SHADED ? 9 : 0);
   constexpr int NT = G_COL + (NEED_COL ? 9 : 0);         // per-face terms
   constexpr int NT1 = NT > 0 ? NT : 1;
-  __shared__ float s_acc[kFaceSlots][NT1];
-  __shared__ int s_face[kFaceSlots];
+  // face slots: 96, or with the colour terms 82, which leave room for four wavefronts per SIMD in the
+  // 160 KB of LDS (200k vertex-coloured faces over 16 x 1024^2, forward + backward 1468 -> 1432 us,
+  // 1445 with 88 and 92).  Fewer than 96 of 18 terms gain nothing (fit_batch of 16 x 4 x 512^2, 70k
+  // faces: 1663 us, with 88, 80 and 72 slots 1665, 1668 and 1674).
+  constexpr int kSlots = NT > 18 ? 82 : 96;
+  __shared__ float s_acc[kSlots][NT1];
+  __shared__ int s_face[kSlots];
+  constexpr int kMergeSlots = NT <= 18 ? 32 : 0;     // flush: slots up to which their corners are merged
+  __shared__ int s_vid[kMergeSlots ? 3 * kMergeSlots : 1];   // flush: the corners' vertices, -1 once summed into another corner
+  __shared__ int s_list[kMergeSlots ? 64 : 1];       // flush: corners left of a batch of 64
   // face id -> slot: open addressing with linear probing, keys face + 1 (0: free)
   __shared__ int2 s_hash[kHashCap];
   constexpr int TS = ALBEDO == kTextured ? 64 : 1;
@@ -358,24 +366,78 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
   for (int k = 0; k < 27; ++k) sh_acc[k] = 0.f;
   bool any = false;
   int nslots = 0;
-  static_assert(kHashCap % 64 == 0 && kHashCap > kFaceSlots, "hash table: whole lanes, spare capacity");
+  static_assert(kHashCap % 64 == 0 && kHashCap > kSlots, "hash table: whole lanes, spare capacity");
 #pragma unroll
   for (int q = 0; q < kHashCap / 64; ++q) s_hash[lane + 64 * q].x = 0;
   __syncthreads();
 
+  // Flush of the slots by lane-parallel global atomics.  Atomics are executed on the memory side, at 16
+  // to 20 G requests/s whatever the scope, and this kernel issues 17 G/s of them (5.3 M in 312 us at
+  // 100k textured faces over 8 x 1024^2), so where it is cheap the requests are reduced first: a vertex
+  // of the tile belongs to several of its faces (six in a regular mesh), and the slots' corners of one
+  // vertex are summed in LDS.  Every corner writes itself to its vertex's entry of a claim table (the
+  // face table's memory: one 8-byte write, the last one stays), the corners whose entry names another
+  // corner of their vertex add their terms to that one's, and the rest (claimants, and vertices whose
+  // entry another vertex took) are flushed, one row of terms per vertex on adjacent lanes.
+  // The LDS additions grow with the faces and the colour terms, so tiles of more than 32 faces, and the
+  // kernel with colour terms, flush slot by slot: forward + backward 632 -> 625 us at 100k textured
+  // faces over 8 x 1024^2 (about 34 faces a tile), 276 -> 253 us at 320 faces over 4 x 1024^2 (where
+  // every tile adds to the same few vertices), 159 -> 156 us at 16k faces over 6 x 333 x 477; merging
+  // every tile takes 1780 us for 1663 at 16 x 4 x 512^2 with 70k faces.
   auto flush = [&]() {
+    constexpr int kComps = NT > 0 ? NT / 3 : 1;           // terms of a corner
     __syncthreads();
-    for (int i = lane; i < nslots * NT; i += 64) {
-      const int slot = i / NT, k = i % NT;
-      const float v = s_acc[slot][k];
-      if (v == 0.f) continue;
-      const int grp = k / 9, kk = k % 9;
-      const int vtx = a.faces[3 * s_face[slot] + kk / 3];
-      const size_t row = (size_t)b * a.N + vtx;
-      float* dst;
-      if (SHADED && grp < 2) dst = a.g_pv + row * 6 + 3 * grp + kk % 3;   // position, normal: one 24-byte row
-      else dst = (grp * 9 == G_POS && NEED_POS ? a.g_pos : a.g_col) + row * 3 + kk % 3;
-      atomicAdd(dst, v);
+    if (nslots > kMergeSlots) {
+      for (int i = lane; i < nslots * NT; i += 64) {
+        const int slot = i / NT1, k = i % NT1;
+        const float v = s_acc[slot][k];
+        if (v == 0.f) continue;
+        const int grp = k / 9, kk = k % 9;
+        const int vtx = a.faces[3 * s_face[slot] + kk / 3];
+        const size_t row = (size_t)b * a.N + vtx;
+        float* dst;
+        if (SHADED && grp < 2) dst = a.g_pv + row * 6 + 3 * grp + kk % 3;   // position, normal: one 24-byte row
+        else dst = (grp * 9 == G_POS && NEED_POS ? a.g_pos : a.g_col) + row * 3 + kk % 3;
+        atomicAdd(dst, v);
+      }
+      nslots = 0;
+    }
+    const int corners = kMergeSlots ? 3 * nslots : 0;
+    for (int c = lane; c < corners; c += 64) {
+      const int v = a.faces[3 * s_face[c / 3] + c % 3];
+      s_vid[c] = v;
+      s_hash[v & (kHashCap - 1)] = make_int2(v, c);
+    }
+    __syncthreads();
+    for (int c = lane; c < corners; c += 64) {
+      const int v = s_vid[c];
+      const int2 o = s_hash[v & (kHashCap - 1)];
+      if (o.x != v || o.y == c) continue;
+      const float* mine = &s_acc[c / 3][3 * (c % 3)];
+      float* to = &s_acc[o.y / 3][3 * (o.y % 3)];
+#pragma unroll
+      for (int m = 0; m < kComps; ++m) atomicAdd(to + 9 * (m / 3) + m % 3, mine[9 * (m / 3) + m % 3]);
+      s_vid[c] = -1;
+    }
+    __syncthreads();
+    for (int c0 = 0; c0 < corners; c0 += 64) {
+      const int c = c0 + lane;
+      const bool left = c < corners && s_vid[c] >= 0;
+      const uint64_t alive = __ballot(left);
+      if (left)
+        s_list[__builtin_amdgcn_mbcnt_hi((unsigned)(alive >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)alive, 0u))] = c;
+      __syncthreads();
+      for (int i = lane; i < __popcll(alive) * kComps; i += 64) {
+        const int r = i / kComps, m = i - r * kComps, grp = m / 3, kk = m - 3 * grp, e = s_list[r];
+        const float v = s_acc[e / 3][9 * grp + 3 * (e % 3) + kk];
+        if (v == 0.f) continue;
+        const size_t row = (size_t)b * a.N + s_vid[e];
+        float* dst;
+        if (SHADED && grp < 2) dst = a.g_pv + row * 6 + 3 * grp + kk;   // position, normal: one 24-byte row
+        else dst = (grp * 9 == G_POS && NEED_POS ? a.g_pos : a.g_col) + row * 3 + kk;
+        atomicAdd(dst, v);
+      }
+      __syncthreads();
     }
 #pragma unroll
     for (int q = 0; q < kHashCap / 64; ++q) s_hash[lane + 64 * q].x = 0;
@@ -398,8 +460,9 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
   int nidf = round_pixel(0, npx, npy, nidx);
   int ni0 = 0, ni1 = 0, ni2 = 0;
   if (nidf >= 0) { ni0 = a.faces[3 * nidf]; ni1 = a.faces[3 * nidf + 1]; ni2 = a.faces[3 * nidf + 2]; }
-  for (int round = 0; round < RT * RT; ++round) {
-    const int px = npx, py = npy, idf = nidf, i0 = ni0, i1 = ni1, i2 = ni2;
+  for (int round = 0;; ++round) {
+    const bool last = round == RT * RT;       // after the rounds: flush only
+    const int px = npx, py = npy, idf = last ? -1 : nidf, i0 = ni0, i1 = ni1, i2 = ni2;
     const size_t idx = nidx;
     if (round + 1 < RT * RT) nidf = round_pixel(round + 1, npx, npy, nidx);
     uint64_t pending = __ballot(idf >= 0);
@@ -444,8 +507,10 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
       }
       __syncthreads();
     }
-    if (!pending) continue;
-    if (NT == 0) continue;
+    if (NT == 0) {
+      if (last) break;
+      continue;
+    }
     // assign each distinct face of this round a slot (reusing slots of earlier rounds).  The
     // round adds at most as many faces as it has runs of equal ids along the lanes (a run
     // starts where a lane's face differs from the previous lane's, or at a 16-lane row start),
@@ -454,8 +519,10 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
     {
       const int prev = __builtin_amdgcn_update_dpp(-2, idf, 0x111, 0xf, 0xf, false);   // row_shr:1
       const int runs = __popcll(__ballot(idf >= 0 && idf != prev));
-      if (nslots + runs > kFaceSlots) flush();
+      if (nslots > 0 && (last || nslots + runs > kSlots)) flush();
     }
+    if (last) break;
+    if (!pending) continue;
     // every lane finds or inserts its face in the hash table at once; the lanes that inserted a
     // face number their new slots in lane order
     int myslot = -1, h = 0;
@@ -495,8 +562,6 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
         if (t[k] != 0.f) atomicAdd(&s_acc[myslot][k], t[k]);
     }
   }
-  if (NT > 0 && nslots > 0) flush();
-
   if (SHADED) {
     // lane 2k stores the tile's total of coefficient k
     const float s = any ? wave_sums27(sh_acc, lane) : 0.f;
