@@ -519,7 +519,11 @@ __global__ __launch_bounds__(64 * kSumLanes) void k_split_sum(const float* __res
 // fp32 master weights [Cout][T][Cin] -> bf16 copy and bf16 transpose [Cin][T][Cout], for up to
 // kPrepareLayers layers in one launch (a launch of its own per layer took 4 us each, 5 to 7 layers
 // of them idle): layer l owns blocks [start[l], start[l + 1]).
-constexpr int kPrepareLayers = 16;
+// Bound by memory (8 bytes a weight; 1.65 M weights 2.6 us at the copy rate) and latency.  A block
+// takes kPrepCo rows x kPrepJ columns of the layer as a matrix [Cout][T * Cin] and turns them in LDS,
+// so that loads and both stores are runs of 64 bytes and more: one thread per weight with its
+// transposed store 2 bytes wide, each to a line of its own, took 13.8 us, this 8.4.
+constexpr int kPrepareLayers = 16, kPrepCo = 32, kPrepJ = 64;
 struct PrepareArgs {
   const float* w[kPrepareLayers];
   uint16_t* wb[kPrepareLayers];
@@ -529,19 +533,42 @@ struct PrepareArgs {
   int n;
 };
 
-__global__ void k_prepare_weights(PrepareArgs a) {
+__global__ __launch_bounds__(256) void k_prepare_weights(PrepareArgs a) {
+  __shared__ uint16_t tile[kPrepJ][kPrepCo + 2];         // rows 17 words apart: no two lanes of a store share a bank
   int l = 0;
   while (l + 1 < a.n && blockIdx.x >= a.start[l + 1]) ++l;
   const int Cout = a.cout[l], T = a.taps[l], Cin = a.cin[l];
-  const int64_t i = int64_t(blockIdx.x - a.start[l]) * blockDim.x + threadIdx.x;
-  const int64_t n = int64_t(Cout) * T * Cin;
-  if (i >= n) return;
-  const int ci = int(i % Cin);
-  const int64_t r = i / Cin;
-  const int t = int(r % T), co = int(r / T);
-  const uint16_t h = f2bf(a.w[l][i]);
-  a.wb[l][i] = h;
-  if (a.wt[l]) a.wt[l][(int64_t(ci) * T + t) * Cout + co] = h;
+  const int64_t row = int64_t(T) * Cin;
+  const unsigned jblocks = unsigned((row + kPrepJ - 1) / kPrepJ), blk = blockIdx.x - a.start[l];
+  const int co0 = int(blk / jblocks) * kPrepCo;
+  const int64_t j0 = int64_t(blk % jblocks) * kPrepJ;
+  {
+    const int dj = threadIdx.x % kPrepJ, r = threadIdx.x / kPrepJ;
+    constexpr int kRows = 256 / kPrepJ, kLoads = kPrepCo / kRows;
+    float v[kLoads];
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) {
+      const int co = co0 + r + kRows * k;
+      v[k] = co < Cout && j0 + dj < row ? a.w[l][co * row + j0 + dj] : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) {
+      const int co = co0 + r + kRows * k;
+      const uint16_t h = f2bf(v[k]);
+      if (co < Cout && j0 + dj < row) a.wb[l][co * row + j0 + dj] = h;
+      tile[dj][co - co0] = h;
+    }
+  }
+  if (!a.wt[l]) return;
+  __syncthreads();
+  const int co = co0 + int(threadIdx.x % kPrepCo);
+  if (co >= Cout) return;
+  const int64_t t0 = j0 / Cin;
+  for (int dj = threadIdx.x / kPrepCo; dj < kPrepJ && j0 + dj < row; dj += 256 / kPrepCo) {
+    int64_t ci = j0 - t0 * Cin + dj, t = t0;              // column of the matrix: tap and input channel
+    while (ci >= Cin) ci -= Cin, ++t;
+    a.wt[l][(ci * T + t) * Cout + co] = tile[dj][co - co0];
+  }
 }
 
 // Renders [B][V][h][w][3] fp32 -> NHWC8 bf16 mosaic [B][rows*h/d][cols*w/d][8]: view v at tile
@@ -653,8 +680,8 @@ int launch(ConvArgs a, hipStream_t s, const char* what) {
 // with four waves, of the 128-channel layer 24 against 28); with fewer, the stretches of the
 // reduction are loaded side by side, all at once where the waves' registers hold them (the 4096-deep
 // head of one image: 13 us with 16 waves, 21 with 8 and two rounds of loads, 75 with one wave; the
-// 2304-deep layer 9.4 us with 8 waves, 11.8 with 16, whose accumulators travel twice as far).  Tiles of 32 x 128 and
-// 64 x 128 were no faster (30 and 30 us for those two).
+// 2304-deep layer 9.4 us with 8 waves, 11.8 with 16, whose accumulators travel twice as far).  Tiles
+// of 32 x 128 and 64 x 128 were no faster (30 and 30 us for those two).
 template <bool FWD>
 int launch_conv(const ConvArgs& a, hipStream_t s, const char* what) {
   const ConvGeom& g = a.g;
@@ -798,7 +825,7 @@ int gvv_conv_prepare_weights_layers(int32_t n, const int32_t* Cout, const int32_
       a.wt[k] = static_cast<uint16_t*>(wt_bf16[l]);
       a.cout[k] = Cout[l]; a.taps[k] = taps[l]; a.cin[k] = Cin[l];
       a.start[k] = unsigned(blocks);
-      blocks += (int64_t(Cout[l]) * taps[l] * Cin[l] + 255) / 256;
+      blocks += ((int64_t(Cout[l]) + kPrepCo - 1) / kPrepCo) * ((int64_t(taps[l]) * Cin[l] + kPrepJ - 1) / kPrepJ);
       if (blocks > INT32_MAX) return gvv::set_last_error("prepare weights: too many weights");
       a.n = k + 1;
       a.start[k + 1] = unsigned(blocks);
