@@ -34,6 +34,7 @@ import numpy as np
 import torch
 
 from . import _lib, fit
+from .renderer import _raw_stream
 
 N_OUT = 113
 N_OUT_PAD = 128
@@ -49,7 +50,7 @@ def _ptr(t):
 
 
 def _stream():
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    return _raw_stream(torch.cuda.current_device())
 
 
 def param_stats(n_basis: int, device):
