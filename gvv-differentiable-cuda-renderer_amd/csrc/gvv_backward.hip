@@ -23,6 +23,7 @@
 //                  plain stores, no atomics.  SH: fixed-order reduction of the SH partials
 //                  (deterministic).
 #include "gvv_bary_grad.hpp"
+#include "gvv_claim.hpp"
 #include "gvv_kernels.hpp"
 
 namespace gvv {
@@ -377,7 +378,7 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
   // it is cheap the requests are reduced first: a vertex
   // of the tile belongs to several of its faces (six in a regular mesh), and the slots' corners of one
   // vertex are summed in LDS.  Every corner writes itself to its vertex's entry of a claim table (the
-  // face table's memory: one 8-byte write, the last one stays), the corners whose entry names another
+  // key words of the face table; gvv_claim.hpp), the corners whose entry names another
   // corner of their vertex add their terms to that one's, and the rest (claimants, and vertices whose
   // entry another vertex took) are flushed, one row of terms per vertex on adjacent lanes.
   // The LDS additions grow with the faces and the colour terms, so tiles of more than 32 faces, and the
@@ -407,15 +408,14 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
     for (int c = lane; c < corners; c += 64) {
       const int v = a.faces[3 * s_face[c / 3] + c % 3];
       s_vid[c] = v;
-      s_hash[v & (kHashCap - 1)] = make_int2(v, c);
+      s_hash[v & (kHashCap - 1)].x = claim_entry(c);
     }
     __syncthreads();
     for (int c = lane; c < corners; c += 64) {
-      const int v = s_vid[c];
-      const int2 o = s_hash[v & (kHashCap - 1)];
-      if (o.x != v || o.y == c) continue;
+      const int o = claim_target(s_hash[s_vid[c] & (kHashCap - 1)].x, s_vid, c);
+      if (o == c) continue;
       const float* mine = &s_acc[c / 3][3 * (c % 3)];
-      float* to = &s_acc[o.y / 3][3 * (o.y % 3)];
+      float* to = &s_acc[o / 3][3 * (o % 3)];
 #pragma unroll
       for (int m = 0; m < kComps; ++m) atomicAdd(to + 9 * (m / 3) + m % 3, mine[9 * (m / 3) + m % 3]);
       s_vid[c] = -1;
