@@ -104,6 +104,7 @@ int plan_forward(Handle* h, int B, int texH, int texW, const float* vpos, const 
   const int64_t pix = (int64_t)B * h->C * h->W * h->H;
   size_t old_keys = h->keys.n;
   GVV_CHECK(h->cams.reserve((size_t)B * h->C));
+  GVV_CHECK(h->view_err.reserve((size_t)B * h->C));
   GVV_CHECK(h->fnormal.reserve((size_t)B * h->F * 3));
   GVV_CHECK(h->tris.reserve((size_t)B * h->F));
   GVV_CHECK(h->proj.reserve((size_t)B * h->C * h->N));
@@ -145,7 +146,7 @@ int plan_forward(Handle* h, int B, int texH, int texW, const float* vpos, const 
   p.vpos = vpos; p.extr = extr; p.intr = intr;
   p.faces = h->d_faces.p; p.csr_start = h->d_csr_start.p; p.csr_count = h->d_csr_count.p; p.csr_list = h->d_csr_list.p;
   p.uv_table = h->d_uv_table.p;
-  p.cams = h->cams.p; p.fnormal = h->fnormal.p; p.tris = h->tris.p; p.proj = h->proj.p;
+  p.cams = h->cams.p; p.view_err = h->view_err.p; p.fnormal = h->fnormal.p; p.tris = h->tris.p; p.proj = h->proj.p;
   p.counters = h->counters.p; p.large = h->large.p; p.large_box = h->large_box;
   p.mesh_id = 0; p.shared_queue = false;
   p.raster_items = (int64_t)B * h->C * h->F;

@@ -32,6 +32,7 @@ __device__ __forceinline__ void setup_body(const SetupGrid& g, int blk) {
       Camera c;
       camera_setup(a.extr + 12 * (size_t)i, a.intr + 9 * (size_t)i, c);
       a.cams[i] = c;
+      if (a.view_err) a.view_err[i] = view_error(c, a.W, a.H);
     }
     return;
   }
@@ -48,7 +49,11 @@ __device__ __forceinline__ void setup_body(const SetupGrid& g, int blk) {
       float* o = a.fnormal + 3 * i;
       o[0] = n.x; o[1] = n.y; o[2] = n.z;
     }
-    if (a.tris) a.tris[i] = tri_setup(v0, v1, v2);
+    if (a.tris) {
+      TriSetup t = tri_setup(v0, v1, v2);
+      t.shape = face_shape(t);
+      a.tris[i] = t;
+    }
     if (a.face_grad) {
       FaceGrad r;
       r.t = tri_setup(v0, v1, v2);
@@ -165,8 +170,9 @@ __device__ __forceinline__ void vertices_body(const VertexArgs& va, int64_t blk)
   if (!valid) return;
   float* o = vnormal + 3 * i;
   o[0] = acc.x; o[1] = acc.y; o[2] = acc.z;
-  const V3 p = project(cams[bc], ld3(vpos + ((size_t)b * N + v) * 3));
-  proj[i] = make_float4(p.x, p.y, p.z, 0.f);
+  const V3 x = ld3(vpos + ((size_t)b * N + v) * 3);
+  const V3 p = project(cams[bc], x);
+  proj[i] = make_float4(p.x, p.y, p.z, vertex_error(va.view_err[bc], x, p));
 }
 
 __global__ void __launch_bounds__(256) k_vertices(VertexArgs va) { vertices_body(va, blockIdx.x); }
@@ -296,7 +302,6 @@ __device__ __forceinline__ void flush_candidates(const FaceStage* st, const Stag
     t.v1 = v3(fs.v[3], fs.v[4], fs.v[5]);
     t.v2 = v3(fs.v[6], fs.v[7], fs.v[8]);
     t.N = v3(fs.v[9], fs.v[10], fs.v[11]);
-    t.den = dot(t.N, t.N);      // as tri_setup forms it; only a subnormal quotient divides by it
     t.rden = fs.rden;
     V3 abc;
     // a and b of a hit are not negative, so that of inside()'s six bounds these three are left
@@ -436,9 +441,9 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
         to_queue = sub == 0;
       } else {
         small = true;
-        if (sub == 0)
-          stage_face(&st[slot], tris[(size_t)(bc / C) * F + f], cam_origin_scaled(cams[bc]), f, r.p0.z, r.p1.z, r.p2.z);
-        et = edge_test(r.p0, r.p1, r.p2);
+        const TriSetup& tri = tris[(size_t)(bc / C) * F + f];
+        if (sub == 0) stage_face(&st[slot], tri, cam_origin_scaled(cams[bc]), f, r.p0.z, r.p1.z, r.p2.z);
+        et = edge_test(r.p0, r.p1, r.p2, tri.shape);
         fx0 = r.bx.x0;
         fy0 = r.bx.y0;
       }
@@ -518,12 +523,12 @@ __device__ __forceinline__ void raster_large_face(const TriSetup* __restrict__ t
   const int bw = r.bx.x1 - r.bx.x0 + 1, bh = r.bx.y1 - r.bx.y0 + 1;
   parts = max(1, min(parts, min(min(bw, bh), (int)(((int64_t)bw * bh) / kLargePart))));
   if (part >= parts) return;
+  const TriSetup& tri = tris[(size_t)(bc / C) * F + f];
   BoxLines bl;
-  bl.start(edge_test(r.p0, r.p1, r.p2), r.bx.x0, r.bx.y0, bw, bh);
+  bl.start(edge_test(r.p0, r.p1, r.p2, tri.shape), r.bx.x0, r.bx.y0, bw, bh);
   const int lane = threadIdx.x & 63;
   wave_sync();
-  if (lane == 0)
-    stage_face(&st[0], tris[(size_t)(bc / C) * F + f], cam_origin_scaled(cams[bc]), f, r.p0.z, r.p1.z, r.p2.z);
+  if (lane == 0) stage_face(&st[0], tri, cam_origin_scaled(cams[bc]), f, r.p0.z, r.p1.z, r.p2.z);
   const StageOwner own{bc, r.bx.x0, r.bx.y0, bw};
   wave_sync();
   const bool packed = cand_packed(W, H);
@@ -723,6 +728,7 @@ static void launch_resolve_t(const ResolveArgs& a, hipStream_t s) {
 SetupArgs forward_setup_args(const ForwardPlan& p) {
   SetupArgs sa;
   sa.extr = p.extr; sa.intr = p.intr; sa.cams = p.cams; sa.n_cams = p.B * p.C;
+  sa.view_err = p.view_err; sa.W = p.r.W; sa.H = p.r.H;
   sa.vpos = p.vpos; sa.faces = p.faces; sa.fnormal = p.fnormal; sa.tris = p.tris;
   sa.B = p.B; sa.N = p.N; sa.F = p.F;
   sa.counters = p.shared_queue ? nullptr : p.counters;
@@ -732,7 +738,7 @@ SetupArgs forward_setup_args(const ForwardPlan& p) {
 VertexArgs vertex_args(const ForwardPlan& p) {
   VertexArgs a;
   a.vpos = p.vpos; a.fnormal = p.fnormal; a.csr_start = p.csr_start; a.csr_count = p.csr_count;
-  a.csr_list = p.csr_list; a.cams = p.cams; a.vnormal = p.vnormal_out; a.proj = p.proj;
+  a.csr_list = p.csr_list; a.cams = p.cams; a.view_err = p.view_err; a.vnormal = p.vnormal_out; a.proj = p.proj;
   a.B = p.B; a.C = p.C; a.N = p.N; a.F = p.F;
   return a;
 }

@@ -41,6 +41,7 @@ struct Handle {
   DevBuf<UvTexel> d_uv_table;
   // scratch
   DevBuf<Camera> cams;
+  DevBuf<ViewError> view_err;          // the pre-test's error terms per view
   DevBuf<float> fnormal;
   DevBuf<TriSetup> tris;
   DevBuf<float4> proj;
@@ -56,7 +57,7 @@ struct Handle {
 
   ~Handle() {
     d_faces.release(); d_csr_start.release(); d_csr_count.release(); d_csr_list.release();
-    d_uv.release(); d_uv_table.release(); cams.release(); fnormal.release(); tris.release(); proj.release();
+    d_uv.release(); d_uv_table.release(); cams.release(); view_err.release(); fnormal.release(); tris.release(); proj.release();
     keys.release(); counters.release(); tile_count.release(); tile_dirty.release(); bins.release(); large.release(); g_pv.release(); sh_partial.release();
     face_grad.release();
   }

@@ -5,6 +5,7 @@
 
 #include "gvv_bary_grad.hpp"
 #include "gvv_math.hpp"
+#include "gvv_raster.hpp"
 
 namespace gvv {
 
@@ -156,8 +157,9 @@ struct VertexArgs {
   const int32_t* csr_count;
   const int32_t* csr_list;
   const Camera* cams;                // [B][C]
+  const ViewError* view_err;         // [B][C]
   float* vnormal;                    // [B][C][N][3]
-  float4* proj;                      // [B][C][N]
+  float4* proj;                      // [B][C][N] projected vertices, vertex_error in w
   int B, C, N, F;
 };
 
@@ -202,6 +204,7 @@ struct ForwardPlan {
   const int32_t* csr_list;
   const UvTexel* uv_table;
   Camera* cams;
+  ViewError* view_err;               // [B][C] the pre-test's error terms
   float* fnormal;                    // [B][F][3]
   TriSetup* tris;                    // [B][F] scaled ray/triangle constants
   float4* proj;                      // [B][C][N]
@@ -292,7 +295,8 @@ struct SetupArgs {
   const float* extr = nullptr;
   const float* intr = nullptr;
   Camera* cams = nullptr;
-  int n_cams = 0;
+  ViewError* view_err = nullptr;     // the forward's (W, H: its image)
+  int n_cams = 0, W = 0, H = 0;
   const float* vpos = nullptr;
   const int32_t* faces = nullptr;
   float* fnormal = nullptr;

@@ -226,8 +226,8 @@ struct alignas(16) TriSetup {
   V3 v0, v1, v2;   // vertices / 1000
   V3 N;            // cross(v1 - v0, v2 - v0)
   float dv0N;      // dot(v0, N)
-  float den;       // dot(N, N)
-  double rden;     // its reciprocal (recip64), for the quotients by den
+  uint32_t shape;  // the stored records of the depth pass: the terms of its pre-test's margin (face_shape)
+  double rden;     // reciprocal of dot(N, N) (recip64), for the quotients by it
 };
 
 GVV_HD TriSetup tri_setup(V3 v0, V3 v1, V3 v2) {
@@ -235,8 +235,8 @@ GVV_HD TriSetup tri_setup(V3 v0, V3 v1, V3 v2) {
   t.v0 = div1000(v0); t.v1 = div1000(v1); t.v2 = div1000(v2);
   t.N = cross(t.v1 - t.v0, t.v2 - t.v0);
   t.dv0N = dot(t.v0, t.N);
-  t.den = dot(t.N, t.N);
-  t.rden = recip64(t.den);
+  t.shape = 0u;
+  t.rden = recip64(dot(t.N, t.N));
   return t;
 }
 
@@ -250,7 +250,8 @@ GVV_HD bool ray_hit(const TriSetup& t, float num, V3 o_s, V3 d, V3& abc) {
   float a = dot(t.N, cross(t.v2 - t.v1, P - t.v1));
   float b = dot(t.N, cross(t.v0 - t.v2, P - t.v2));
   const bool miss = fabsf(ndr) < 0.0000001f || tt < 0 || s < 0 || a < 0 || b < 0;
-  a = quot(a, t.den, t.rden); b = quot(b, t.den, t.rden);
+  const float den = dot(t.N, t.N);      // only a subnormal quotient divides by it
+  a = quot(a, den, t.rden); b = quot(b, den, t.rden);
   abc = v3(a, b, 1.f - a - b);
   return !miss;
 }

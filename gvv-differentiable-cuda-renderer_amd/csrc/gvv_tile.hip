@@ -61,6 +61,7 @@ __device__ __forceinline__ int next_tile(const EdgeTest& et, int k, int n, int t
 }
 
 __global__ void __launch_bounds__(256) k_bin(const int32_t* __restrict__ faces, const float4* __restrict__ proj,
+                                             const TriSetup* __restrict__ tris,
                                              unsigned* __restrict__ tile_count, unsigned* __restrict__ bins,
                                              unsigned int* __restrict__ large_count, int4* __restrict__ large, int B,
                                              int C, int N, int F, int W, int H, TileMarks tm, int mesh_id) {
@@ -87,7 +88,7 @@ __global__ void __launch_bounds__(256) k_bin(const int32_t* __restrict__ faces, 
         to_queue = true;
         n = 0;
       } else {
-        et = edge_test(p0, p1, p2);
+        et = edge_test(p0, p1, p2, tris[(size_t)(bc / C) * F + f].shape);
         k = next_tile(et, 0, n, tw, tx0, ty0, W, H, tm.sx, tm.sy);
       }
     }
@@ -223,7 +224,7 @@ __global__ void __launch_bounds__(256) k_tile(TileArgs a) {
           s.z0 = p0.z; s.z1 = p1.z; s.z2 = p2.z;
           s.f = f;
           st[lane] = s;
-          et = edge_test(p0, p1, p2);
+          et = edge_test(p0, p1, p2, s.t.shape);
         } else {
           bw = bh = 0;
         }
@@ -308,7 +309,7 @@ static void launch_tile_t(const TileArgs& a, int sx, int sy, int64_t n, hipStrea
 hipError_t launch_bin(const ForwardPlan& p, hipStream_t s) {
   const int64_t n = (int64_t)p.B * p.C * p.F;
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_bin, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p.faces, p.proj, p.tile_count, p.bins,
+  hipLaunchKernelGGL(k_bin, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p.faces, p.proj, p.tris, p.tile_count, p.bins,
                      p.counters, p.large, p.B, p.C, p.N, p.F, p.r.W, p.r.H, p.marks, p.mesh_id);
   return hipGetLastError();
 }

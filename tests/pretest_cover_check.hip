@@ -1,0 +1,149 @@
+// The depth pass's pre-test with the margin that the kernels give it (gvv_raster.hpp view_error,
+// vertex_error, face_shape, edge_test) against the exact ray/triangle test, over faces whose own
+// binary32 errors are large: needles, vertices from 1 mm in front of the camera, vertices far off
+// screen, long lenses, wide images and scenes far from the world's origin, at every orientation.
+// Boxes are of any size; on every line of a box the exact test is run on the pixels around both ends
+// of the span (or, where the span is empty, around the place where the edges are nearest), outside
+// it only.  Per class: the accepted pixels outside the spans (missed) and outside the three half-planes
+// of the direct test (missed_px), the same with kEdgeMargin alone (plain), the faces with the pre-test
+// on, and the largest share of a face's bound that an accepted pixel needed.  Host only.
+#include <algorithm>
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <random>
+#include "../gvv-differentiable-cuda-renderer_amd/csrc/gvv_raster.hpp"
+using namespace gvv;
+
+int main(int argc, char** argv) {
+  const int n = argc > 1 ? atoi(argv[1]) : 2000;
+  const int seed = argc > 2 ? atoi(argv[2]) : 5;
+  const char* names[] = {"ordinary", "needles", "near", "closeup", "offscreen", "lens", "far"};
+  for (int cls = 0; cls < 7; ++cls) {
+    std::mt19937 rng(seed * 100 + cls);
+    std::uniform_real_distribution<double> U(0, 1);
+    std::normal_distribution<double> G(0, 1);
+    auto logu = [&](double a, double b) { return a * std::pow(b / a, U(rng)); };
+    long long missed = 0, missed_px = 0, plain = 0, on = 0, faces = 0, accepted = 0;
+    double share = 0;
+    for (int t = 0; t < n; ++t) {
+      int W = 1024, H = t % 3 ? 1024 : 389;
+      double f = 1.2 * W;
+      if (cls == 5) { W = t % 2 ? 8192 : 1024; H = t % 3 ? W : W / 3; f = W * logu(0.5, 20); }
+      // a random rotation and a camera position; the points are drawn in camera coordinates
+      double q[4], nq = 0;
+      for (double& x : q) { x = G(rng); nq += x * x; }
+      for (double& x : q) x /= std::sqrt(nq);
+      if (t % 4 == 0) { q[0] = 1; q[1] = q[2] = q[3] = 0; }
+      const double R[9] = {1 - 2 * (q[2] * q[2] + q[3] * q[3]), 2 * (q[1] * q[2] - q[0] * q[3]), 2 * (q[1] * q[3] + q[0] * q[2]),
+                           2 * (q[1] * q[2] + q[0] * q[3]), 1 - 2 * (q[1] * q[1] + q[3] * q[3]), 2 * (q[2] * q[3] - q[0] * q[1]),
+                           2 * (q[1] * q[3] - q[0] * q[2]), 2 * (q[2] * q[3] + q[0] * q[1]), 1 - 2 * (q[1] * q[1] + q[2] * q[2])};
+      double pos[3] = {G(rng) * 2000, G(rng) * 500, G(rng) * 2000};
+      if (cls == 6) for (double& x : pos) x *= logu(10, 1000);
+      float E[12], K[9] = {(float)f, t % 5 == 1 ? 3.f : 0.f, (float)(W * (0.3 + 0.4 * U(rng))), 0, (float)(f * (0.9 + 0.2 * U(rng))),
+                           (float)(H * (0.3 + 0.4 * U(rng))), 0, 0, 1};
+      for (int r = 0; r < 3; ++r) {
+        double s = 0;
+        for (int c = 0; c < 3; ++c) { E[4 * r + c] = (float)R[3 * r + c]; s += (double)E[4 * r + c] * pos[c]; }
+        E[4 * r + 3] = (float)-s;
+      }
+      Camera cam;
+      camera_setup(E, K, cam);
+      const ViewError ve = view_error(cam, W, H);
+      // the point that camera coordinates (x, y, z) name, in world coordinates
+      auto world = [&](const double* c, V3& out) {
+        double w[3];
+        for (int k = 0; k < 3; ++k) w[k] = pos[k] + R[k] * c[0] + R[3 + k] * c[1] + R[6 + k] * c[2];
+        out = v3((float)w[0], (float)w[1], (float)w[2]);
+      };
+      auto at_pixel = [&](double x, double y, double z, double* c) {
+        c[2] = z;
+        c[1] = (y - K[5]) / K[4] * z;
+        c[0] = (x - K[2] - K[1] * c[1] / z) / K[0] * z;
+      };
+      double c[3][3];
+      const double depth = cls == 6 ? logu(500, 50000) : 600 + 4400 * U(rng);
+      for (int k = 0; k < 3; ++k) {
+        double z = depth * (1 + 0.05 * G(rng)), x, y;
+        if (cls == 2) z = 50 + 3000 * U(rng);
+        if (cls == 3) z = logu(1.0, 5000);
+        const double px = cls == 2 || cls == 3 || cls == 4 ? W : logu(3, W);
+        x = W / 2. + (k == 0 ? (U(rng) - 0.5) * W : 0) + G(rng) * px * 0.4;
+        y = H / 2. + (k == 0 ? (U(rng) - 0.5) * H : 0) + G(rng) * px * 0.4;
+        if (k && (cls == 0 || cls == 5 || cls == 6)) { x += (c[0][0] / c[0][2]) * K[0]; y += (c[0][1] / c[0][2]) * K[4]; }
+        if (cls == 4 && k == t % 3) {
+          const double far = logu(2000, t % 2 ? 60000 : 900000), a = 6.2831853 * U(rng);
+          x = far * std::cos(a);
+          y = far * std::sin(a);
+          z = logu(2, 3000);
+        }
+        at_pixel(x, y, std::max(z, 1.0), c[k]);
+      }
+      if (cls == 1) {                 // the third vertex 0.02 .. 1 mm off the line of the other two
+        const double a = U(rng) * 1.2 - 0.1, off = logu(0.02, 1.0);
+        for (int k = 0; k < 3; ++k) c[2][k] = c[0][k] + a * (c[1][k] - c[0][k]) + off * G(rng) * 0.6;
+      }
+      V3 v[3];
+      float4 p[3], p_plain[3];
+      for (int k = 0; k < 3; ++k) {
+        world(c[(k + t) % 3], v[k]);
+        const V3 pr = project(cam, v[k]);
+        p[k] = make_float4(pr.x, pr.y, pr.z, vertex_error(ve, v[k], pr));
+        p_plain[k] = make_float4(pr.x, pr.y, pr.z, 0.f);
+      }
+      const Box bx = face_box(v3(p[0].x, p[0].y, p[0].z), v3(p[1].x, p[1].y, p[1].z), v3(p[2].x, p[2].y, p[2].z), W, H);
+      if (bx.x0 > bx.x1 || bx.y0 > bx.y1) continue;
+      const int bw = bx.x1 - bx.x0 + 1, bh = bx.y1 - bx.y0 + 1;
+      ++faces;
+      const TriSetup ts = tri_setup(v[0], v[1], v[2]);
+      const EdgeTest et = edge_test(p[0], p[1], p[2], face_shape(ts));
+      // the three edges without a margin, in binary64
+      const EdgeTest ep = edge_test(p_plain[0], p_plain[1], p_plain[2]);
+      if (et.on) ++on;
+      if (!ep.on) continue;
+      double ed[3][3];
+      for (int i = 0; i < 3; ++i) {
+        ed[i][0] = ep.a[i];
+        ed[i][1] = ep.b[i];
+        ed[i][2] = -((double)ep.a[i] * p[i].x + (double)ep.b[i] * p[i].y);
+      }
+      const double bound = et.on ? (double)et.c[0] - ed[0][2] : 1e30;      // this face's margin
+      BoxLines bl;
+      bl.start(et, bx.x0, bx.y0, bw, bh);
+      const int step = std::max(1, bl.lines / 256);
+      for (int ln = (int)(rng() % step); ln < bl.lines; ln += step) {
+        int first;
+        const int cnt = bl.span(ln, first);
+        if (cnt < 0 || (cnt > 0 && (first < 0 || first + cnt > bl.len))) { printf("bad span\n"); return 1; }
+        // where the edges leave this line, in binary64
+        double lo = 0, hi = bl.len - 1;
+        for (int i = 0; i < 3; ++i) {
+          const double ea = bl.columns ? ed[i][1] : ed[i][0];
+          const double x = bx.x0 + 0.5 + (bl.columns ? ln : 0), y = bx.y0 + 0.5 + (bl.columns ? 0 : ln);
+          const double b = -(ed[i][0] * x + ed[i][1] * y + ed[i][2]) / ea;
+          if (ea > 0) lo = std::max(lo, b);
+          if (ea < 0) hi = std::min(hi, b);
+        }
+        int at[2] = {(int)std::floor(std::min(std::max(lo, 0.0), bl.len - 1.0)), (int)std::ceil(std::min(std::max(hi, 0.0), bl.len - 1.0))};
+        for (int side = 0; side < 2; ++side)
+          for (int d = -10; d <= 10; ++d) {
+            const int k = at[side] + d;
+            if (k < 0 || k >= bl.len || (side == 1 && std::abs(k - at[0]) <= 10)) continue;
+            const int x = bx.x0 + (bl.columns ? ln : k), y = bx.y0 + (bl.columns ? k : ln);
+            const V3 abc = ray_barycentric(ts, cam_origin_scaled(cam), pixel_ray(cam, x + 0.5f, y + 0.5f));
+            if (!inside(abc)) continue;
+            ++accepted;
+            missed += k < first || k >= first + cnt;
+            missed_px += !et.pass(x + 0.5f, y + 0.5f);
+            plain += !ep.pass(x + 0.5f, y + 0.5f);
+            double need = 0;
+            for (int i = 0; i < 3; ++i) need = std::max(need, -(ed[i][0] * (x + 0.5) + ed[i][1] * (y + 0.5) + ed[i][2]));
+            if (et.on) share = std::max(share, need / bound);
+          }
+      }
+    }
+    printf("%s faces %lld on %lld accepted %lld missed %lld missed_px %lld plain %lld share %.3f\n", names[cls], faces, on, accepted,
+           missed, missed_px, plain, share);
+  }
+  return 0;
+}
