@@ -509,11 +509,15 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) k_
   raster_body<1>(a, m.local);
 }
 
-// Part `part` of `parts` of one large face (bc, f), rasterised by the whole wavefront: lines part,
-// part + parts, ... of its box.  The spans of 64 lines are found at once, one per lane
+// Part `part` of `parts` of one large face (bc, f), rasterised by the whole wavefront: rows part,
+// part + parts, ... of its box.  The spans of 64 rows are found at once, one per lane
 // (BoxLines).  They go to the candidate list one span at a time, 64 pixels per step, or, where
 // they are shorter than they are many (a sliver across its box), all at once, one pixel of each
 // per step.  Full lists take the exact test as in k_raster.
+// Rows also of tall boxes: the pass is bound by the memory side's atomic requests, one per 64-byte line
+// of keys and instruction, and 64 candidates along a column are 64 lines.  With the columns of tall
+// boxes it took 341 us at 2,400 tall faces (about 10 x 70 px) over 8 x 1024^2 and takes 141 with rows,
+// 146 -> 65 us at 320 faces over 4 x 1024^2.
 __device__ __forceinline__ void raster_large_face(const TriSetup* __restrict__ tris, const int32_t* __restrict__ faces,
                                                   const float4* __restrict__ proj, const Camera* __restrict__ cams,
                                                   unsigned long long* __restrict__ keys, int C, int N, int F, int W,
@@ -521,19 +525,18 @@ __device__ __forceinline__ void raster_large_face(const TriSetup* __restrict__ t
                                                   unsigned* cand, TileMarks marks) {
   const RasterFace r = load_face(faces, proj + (size_t)bc * N, f, W, H);
   const int bw = r.bx.x1 - r.bx.x0 + 1, bh = r.bx.y1 - r.bx.y0 + 1;
-  parts = max(1, min(parts, min(min(bw, bh), (int)(((int64_t)bw * bh) / kLargePart))));
+  parts = max(1, min(parts, min(bh, (int)(((int64_t)bw * bh) / kLargePart))));
   if (part >= parts) return;
   const TriSetup& tri = tris[(size_t)(bc / C) * F + f];
   BoxLines bl;
-  bl.start(edge_test(r.p0, r.p1, r.p2, tri.shape), r.bx.x0, r.bx.y0, bw, bh);
+  bl.start_rows(edge_test(r.p0, r.p1, r.p2, tri.shape), r.bx.x0, r.bx.y0, bw, bh);
   const int lane = threadIdx.x & 63;
   wave_sync();
   if (lane == 0) stage_face(&st[0], tri, cam_origin_scaled(cams[bc]), f, r.p0.z, r.p1.z, r.p2.z);
   const StageOwner own{bc, r.bx.x0, r.bx.y0, bw};
   wave_sync();
   const bool packed = cand_packed(W, H);
-  const unsigned step = cand_word(packed, true, 0, bl.columns ? 0 : 1, bl.columns ? 1 : 0, bl.columns ? 0 : 1,
-                                  bl.columns ? 1 : 0, bw);
+  const unsigned step = cand_word(packed, true, 0, 1, 0, 1, 0, bw);
   int count = 0;
   const auto flush = [&](int n) {
     flush_candidates<1>(st, own, cand, n, cams, true, bc, keys, W, H, true, marks);
@@ -542,8 +545,7 @@ __device__ __forceinline__ void raster_large_face(const TriSetup* __restrict__ t
     const int ln = l0 + lane * parts;
     int first = 0;
     const int len = ln < bl.lines ? bl.span(ln, first) : 0;
-    const int dx = bl.columns ? ln : first, dy = bl.columns ? first : ln;
-    const unsigned word = cand_word(packed, true, 0, r.bx.x0 + dx, r.bx.y0 + dy, dx, dy, bw);
+    const unsigned word = cand_word(packed, true, 0, r.bx.x0 + first, r.bx.y0 + ln, first, ln, bw);
     uint64_t todo = __ballot(len > 0);
     const int incl = wave_inclusive_sum(len), total = __builtin_amdgcn_readlane(incl, 63), spans = __popcll(todo);
     if (2 * total <= spans * spans) {

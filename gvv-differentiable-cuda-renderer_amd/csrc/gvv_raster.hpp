@@ -230,7 +230,7 @@ struct EdgeWalk {
 };
 
 // The pixels of a box that the pre-test keeps, line by line: lines run along the box's longer
-// side (rows, or columns of a tall box), and on each line the kept pixels are one interval,
+// side (rows, or columns of a tall box: start) or along its rows (start_rows), and on each line the kept pixels are one interval,
 // because each edge bounds the position along the line from one side.  An edge's bound moves
 // linearly from line to line (t + ln * s), so a line costs three FMAs instead of three edge
 // values per pixel.
@@ -245,8 +245,12 @@ struct BoxLines {
   bool lower[3], upper[3];     // which side it bounds
   int lines, len;              // lines of the box and pixels per line
   bool columns;                // lines are columns (the box is taller than wide)
-  GVV_HD void start(const EdgeTest& e, int x0, int y0, int bw, int bh) {
-    columns = bh > bw;
+  GVV_HD void start(const EdgeTest& e, int x0, int y0, int bw, int bh) { start_lines(e, x0, y0, bw, bh, bh > bw); }
+  // rows of any box, for faces of many pixels: along a row 8 visibility keys share a 64-byte line of
+  // memory, along a column each has its own
+  GVV_HD void start_rows(const EdgeTest& e, int x0, int y0, int bw, int bh) { start_lines(e, x0, y0, bw, bh, false); }
+  GVV_HD void start_lines(const EdgeTest& e, int x0, int y0, int bw, int bh, bool by_columns) {
+    columns = by_columns;
     lines = columns ? bw : bh;
     len = columns ? bh : bw;
     const float x = x0 + 0.5f, y = y0 + 0.5f;
