@@ -409,6 +409,19 @@ __device__ __forceinline__ void append_spans(unsigned* cand, int& count, int rem
 // of the 21 G/s that scattered atomics reach (the large-face pass the same, 0.72 M in 38 us), with
 // VALU issue at 60% (51 M instructions).  Reading a pixel's key before the exact test, to skip the
 // atomic where the face cannot win, adds a memory-side request for each it saves: 165 us.
+// Appends the lanes' faces with `large` set to the large-face queue, with one atomic per wavefront.
+__device__ __forceinline__ void queue_large(const RasterArgs& ra, bool large, int bc, int f) {
+  const uint64_t qm = __ballot(large);
+  if (!qm) return;
+  unsigned int base = 0;
+  if ((int)(threadIdx.x & 63) == __ffsll((unsigned long long)qm) - 1) base = atomicAdd(ra.large_count, (unsigned)__popcll(qm));
+  base = __builtin_amdgcn_readlane(base, __ffsll((unsigned long long)qm) - 1);
+  if (large) {
+    const unsigned off = __builtin_amdgcn_mbcnt_hi((unsigned)(qm >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)qm, 0u));
+    ra.large[base + off] = make_int4(bc, f, ra.mesh_id, 0);
+  }
+}
+
 template <int G>
 __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
   constexpr int kFaces = 64 / G;
@@ -417,14 +430,31 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
   const float4* __restrict__ proj = ra.proj;
   const Camera* __restrict__ cams = ra.cams;
   unsigned long long* __restrict__ keys = ra.keys;
-  unsigned int* __restrict__ large_count = ra.large_count;
-  int4* __restrict__ large = ra.large;
-  const int B = ra.B, C = ra.C, N = ra.N, F = ra.F, W = ra.W, H = ra.H, large_box = ra.large_box, mesh_id = ra.mesh_id;
+  const int B = ra.B, C = ra.C, N = ra.N, F = ra.F, W = ra.W, H = ra.H, large_box = ra.large_box;
   __shared__ FaceStage st[kFaces];
   __shared__ unsigned cand[kCandCap];
   const int lane = threadIdx.x, slot = lane / G, sub = lane % G;
+  const int64_t items = (int64_t)B * C * F;
+  // Large faces go to the queue 64 items at a time whatever G: the queue's cursor is one word on the
+  // memory side, which takes an atomic each 6 to 11 ns, so with an atomic per wavefront of 4 faces a
+  // mesh whose faces are mostly large waited for it (64,000 faces of about 6 x 40 px: 171 us, 31 now;
+  // 19,200 of 10 x 70 px 64 and 12).
+  // With several lanes to a face every G-th wavefront looks at the boxes of its own and the next
+  // G - 1 wavefronts' faces, one lane to a face.
+  if (G > 1 && wg % G == 0) {
+    const int64_t q = wg * kFaces + lane;
+    bool big = false;
+    int qf = 0, qbc = 0;
+    if (q < items) {
+      qf = (int)(q % F);
+      qbc = (int)(q / F);
+      const Box bx = load_face(faces, proj + (size_t)qbc * N, qf, W, H).bx;
+      big = bx.x0 <= bx.x1 && bx.y0 <= bx.y1 && (int64_t)(bx.x1 - bx.x0 + 1) * (bx.y1 - bx.y0 + 1) > large_box;
+    }
+    queue_large(ra, big, qbc, qf);
+  }
   const int64_t i = wg * kFaces + slot;
-  const bool in_range = i < (int64_t)B * C * F;
+  const bool in_range = i < items;
   const int f = in_range ? (int)(i % F) : 0;
   const int bc = in_range ? (int)(i / F) : 0;
   bool small = false, to_queue = false;
@@ -438,7 +468,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
       bw = r.bx.x1 - r.bx.x0 + 1;
       bh = r.bx.y1 - r.bx.y0 + 1;
       if ((int64_t)bw * bh > large_box) {
-        to_queue = sub == 0;
+        to_queue = G == 1;
       } else {
         small = true;
         const TriSetup& tri = tris[(size_t)(bc / C) * F + f];
@@ -449,18 +479,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
       }
     }
   }
-  // large faces go to the queue with one atomic per wavefront (the cursor is a single word
-  // that every wavefront of the launch would otherwise hit once per face)
-  const uint64_t qm = __ballot(to_queue);
-  if (qm) {
-    unsigned int base = 0;
-    if (lane == __ffsll((unsigned long long)qm) - 1) base = atomicAdd(large_count, (unsigned)__popcll(qm));
-    base = __builtin_amdgcn_readlane(base, __ffsll((unsigned long long)qm) - 1);
-    if (to_queue) {
-      const unsigned off = __builtin_amdgcn_mbcnt_hi((unsigned)(qm >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)qm, 0u));
-      large[base + off] = make_int4(bc, f, mesh_id, 0);
-    }
-  }
+  if (G == 1) queue_large(ra, to_queue, bc, f);
   if (!__ballot(small)) return;
   const int bc0 = __builtin_amdgcn_readfirstlane(bc);
   const bool one_view = __ballot(bc != bc0 && in_range) == 0;
