@@ -188,18 +188,6 @@ __global__ void __launch_bounds__(256) k_vertices_multi(MeshTable<VertexArgs> t)
 constexpr unsigned kLargeWaves = 8192;           // persistent wavefronts of the large-face pass
 constexpr unsigned kLargeItems = 8192;          // face parts that a short queue is split into
 constexpr int kLargePart = 512;                   // box pixels below which a large face is not split further
-// (view, face) items up to which the depth pass gives 16, 8 or 2 lanes to a face instead of one.
-// A wavefront's time is a serial chain over its faces' lines and candidates, so with fewer than
-// about 4096 wavefronts the chain, not the chip, is the kernel's time: 20,480 items (4 x 256^2
-// sphere) took 126 us with one lane and 15 us with 16 lanes to a face; 245,760 items (12 views of
-// 517 x 389) forward alone 172 us with one lane, 146, 134 and 127 with 2, 4 and 8.  Further up the
-// lanes of a face still pay by the smaller staging area (one lane to a face holds 64 staged faces
-// and 6 wavefronts per SIMD, two lanes 8): 800,000 items forward + backward 647 us with one lane,
-// 631, 629 and 655 with 2, 4 and 8; then the setup that they repeat outweighs it (3.2 M items 1468,
-// 1475, 1531 us; 4.5 M items 1744, 1769, 1838 us).  The meshes of a multi-mesh run fill the chip
-// together, so their items count together (8 uneven meshes, choosing each by its own 2.10 ms,
-// together 1.56 with one lane, 1.54, 1.56 and 1.63 with 2, 4 and 8).
-constexpr int64_t kRasterItems16 = 65536, kRasterItems8 = 262144, kRasterItems2 = 2097152;
 
 struct RasterFace {
   int f, i0, i1, i2;
@@ -525,7 +513,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) k_
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) k_raster_multi(MeshTable<RasterArgs> t) {
   const MeshSlice m = t.find((unsigned)xcd_contiguous(blockIdx.x, gridDim.x));
   const RasterArgs a = t.load(m.mesh);
-  raster_body<1>(a, m.local);
+  raster_body<kBatchedLanes>(a, m.local);
 }
 
 // Part `part` of `parts` of one large face (bc, f), rasterised by the whole wavefront: rows part,
@@ -794,7 +782,7 @@ hipError_t launch_raster_large_multi(const RasterMesh* meshes, unsigned int* cou
 
 static void launch_raster(const ForwardPlan& p, const RasterArgs& ra, hipStream_t s) {
   const int64_t items = (int64_t)ra.B * ra.C * ra.F;
-  const int g = p.raster_items <= kRasterItems16 ? 16 : p.raster_items <= kRasterItems8 ? 8 : p.raster_items <= kRasterItems2 ? 2 : 1;
+  const int g = raster_lanes(p.raster_items);
   const dim3 grid(blocks_for(items, 64 / g));
   if (g == 16) hipLaunchKernelGGL(k_raster<16>, grid, dim3(64), 0, s, ra);
   else if (g == 8) hipLaunchKernelGGL(k_raster<8>, grid, dim3(64), 0, s, ra);

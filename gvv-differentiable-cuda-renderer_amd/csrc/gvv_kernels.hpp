@@ -190,6 +190,28 @@ struct ResolveArgs {
   float* render;                     // [B][C][H][W][3]
 };
 
+// (view, face) items up to which the depth pass gives 16, 8 or 2 lanes to a face instead of one.
+// A wavefront's time is a serial chain over its faces' lines and candidates, so with fewer than
+// about 4096 wavefronts the chain, not the chip, is the kernel's time: 20,480 items (4 x 256^2
+// sphere) took 126 us with one lane and 15 us with 16 lanes to a face; 245,760 items (12 views of
+// 517 x 389) forward alone 172 us with one lane, 146, 134 and 127 with 2, 4 and 8.  Further up the
+// lanes of a face still pay by the smaller staging area (one lane to a face holds 64 staged faces
+// and 6 wavefronts per SIMD, two lanes 8): 800,000 items forward + backward 647 us with one lane,
+// 631, 629 and 655 with 2, 4 and 8; then the setup that they repeat outweighs it (3.2 M items 1468,
+// 1475, 1531 us; 4.5 M items 1744, 1769, 1838 us).  The meshes of a multi-mesh run fill the chip
+// together, so their items count together (8 uneven meshes, choosing each by its own 2.10 ms,
+// together 1.56 with one lane, 1.54, 1.56 and 1.63 with 2, 4 and 8).
+constexpr int64_t kRasterItems16 = 65536, kRasterItems8 = 262144, kRasterItems2 = 2097152;
+constexpr int raster_lanes(int64_t items) {
+  return items <= kRasterItems16 ? 16 : items <= kRasterItems8 ? 8 : items <= kRasterItems2 ? 2 : 1;
+}
+// One launch over the meshes of a batched multi-mesh run has one variant, one lane to a face.
+constexpr int kBatchedLanes = 1;
+// What a multi-mesh run, and the autotuner's trials of its meshes, choose the lanes by, so that both
+// run the same variant: every mesh's items, or in a batched run the count that takes kBatchedLanes.
+constexpr int64_t shared_raster_items(int64_t items, bool batched) { return batched ? kRasterItems2 + 1 : items; }
+static_assert(raster_lanes(shared_raster_items(0, true)) == kBatchedLanes, "batched runs and their trials");
+
 struct ForwardPlan {
   int B, C, N, F;
   int albedo;

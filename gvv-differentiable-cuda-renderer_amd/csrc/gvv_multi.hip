@@ -269,7 +269,7 @@ int plan_all(Multi* m, const gvv_mesh_io* io, bool backward, hipStream_t s, std:
     fp[i].large = m->large.p;
     fp[i].mesh_id = i;
     fp[i].shared_queue = true;
-    fp[i].raster_items = (int64_t)queue;
+    fp[i].raster_items = shared_raster_items((int64_t)queue, m->batched);
     t[i] = raster_mesh(fp[i]);
   }
   if (m->host_table.size() != t.size() ||
@@ -476,7 +476,8 @@ int gvv_multi_autotune(void* handle, const gvv_mesh_io* io, int32_t reps, void* 
   MULTI_CHECK(hipEventCreate(&b));
   int rc = 0;
   const int n = (int)m->meshes.size();
-  // the trials use the lanes per face of the runs: alone, a mesh would be given more, with which the
+  // the trials use the lanes per face of the runs (in a batched run one, whatever the items): alone, a
+  // mesh would be given more, with which the
   // high thresholds look best (32 meshes of 2k to 200k faces: graph 9.05 ms with the settings so
   // chosen, 7.83 with the defaults)
   int64_t items = 0;
@@ -497,7 +498,7 @@ int gvv_multi_autotune(void* handle, const gvv_mesh_io* io, int32_t reps, void* 
         ForwardPlan fp;
         BackwardPlan bp;
         if (plan_mesh(m, rep, io[rep], true, s, fp, bp)) { rc = 1; break; }
-        fp.raster_items = items;
+        fp.raster_items = shared_raster_items(items, m->batched);
         hipError_t e = enqueue_mesh(fp, bp, true, s);   // warm-up
         float t_min = 1e30f;
         for (int r = 0; r < reps && e == hipSuccess; ++r) {
