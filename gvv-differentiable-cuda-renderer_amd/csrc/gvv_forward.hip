@@ -461,7 +461,7 @@ __device__ __forceinline__ void raster_body(const RasterArgs& ra, int64_t wg) {
         small = true;
         const TriSetup& tri = tris[(size_t)(bc / C) * F + f];
         if (sub == 0) stage_face(&st[slot], tri, cam_origin_scaled(cams[bc]), f, r.p0.z, r.p1.z, r.p2.z);
-        et = edge_test(r.p0, r.p1, r.p2, tri.shape);
+        et = edge_test(r.p0, r.p1, r.p2, tri.shape, r.bx);
         fx0 = r.bx.x0;
         fy0 = r.bx.y0;
       }
@@ -536,7 +536,7 @@ __device__ __forceinline__ void raster_large_face(const TriSetup* __restrict__ t
   if (part >= parts) return;
   const TriSetup& tri = tris[(size_t)(bc / C) * F + f];
   BoxLines bl;
-  bl.start_rows(edge_test(r.p0, r.p1, r.p2, tri.shape), r.bx.x0, r.bx.y0, bw, bh);
+  bl.start_rows(edge_test(r.p0, r.p1, r.p2, tri.shape, r.bx), r.bx.x0, r.bx.y0, bw, bh);
   const int lane = threadIdx.x & 63;
   wave_sync();
   if (lane == 0) stage_face(&st[0], tri, cam_origin_scaled(cams[bc]), f, r.p0.z, r.p1.z, r.p2.z);

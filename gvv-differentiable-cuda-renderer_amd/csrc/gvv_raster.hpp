@@ -32,12 +32,17 @@ namespace gvv {
 //   projection   7 u (|K| (|E| |V| + |t|)) / z per vertex; a point of the triangle moves by no more
 //                than its vertices, so an edge does too
 //   edge values  coefficients and evaluation: 38 u times the largest coordinate
+// All but the last are sums over the vertices weighted by the point's barycentrics in the image, so
+// their maximum bounds them; where that is above kEdgeMargin, the weights are bounded over the box
+// (a vertex far off screen, whose own error may be hundreds of px, moves the edges on the screen by
+// a small share of it: 4,000 faces that each reach to 1.5-20 mm from the camera, 4 views of 512^2,
+// forward 8.8 ms by the maximum alone, 5.5 ms so, 7.1 with the fixed margin, which loses pixels).
 // A projected triangle thinner than its vertices' errors (seen edge-on) can turn its edges by any
 // angle; there a point within the half-planes has barycentrics above -10 u q, in the image up to
 // zr = zmax / zmin times as much, of a height of at most its longest edge.
 // The pre-test is disabled (every bounding-box pixel takes the exact test) when a vertex is near
-// or behind the camera plane, coordinates are beyond 1e6 px, the projected triangle is degenerate,
-// or q zr > 1e5, from where the bound's own terms no longer hold.
+// or behind the camera plane, coordinates are beyond 1e6 px, the projected triangle is degenerate (the
+// sign of its area uncertain), or q zr > 1e5, from where the bound's own terms no longer hold.
 // Each bound is an upper one of sums that mostly cancel; tests/pretest_cover_check.hip draws the
 // cases above and finds accepted pixels out to 0.22 of a face's margin (with kEdgeMargin alone, up to
 // one accepted pixel in 260 is lost there).  At 1024 px, f = 1229 px and cameras 3 to 3.5 m away the
@@ -161,8 +166,9 @@ struct EdgeTest {
   }
 };
 
-// p: projected vertices with vertex_error in w (0: no error); shape: face_shape of the face.
-GVV_HD EdgeTest edge_test(float4 p0, float4 p1, float4 p2, uint32_t shape = 0u) {
+// p: projected vertices with vertex_error in w (0: no error); shape: face_shape of the face; box: the
+// pixels in question.
+GVV_HD EdgeTest edge_test(float4 p0, float4 p1, float4 p2, uint32_t shape, const Box& box) {
   EdgeTest e;
   e.on = false;
   const float px[3] = {p0.x, p1.x, p2.x}, py[3] = {p0.y, p1.y, p2.y}, pz[3] = {p0.z, p1.z, p2.z};
@@ -173,39 +179,61 @@ GVV_HD EdgeTest edge_test(float4 p0, float4 p1, float4 p2, uint32_t shape = 0u) 
   }
   const float area2 = (px[1] - px[0]) * (py[2] - py[0]) - (py[1] - py[0]) * (px[2] - px[0]);
   if (!(fabsf(area2) >= 1e-3f)) return e;
-  float ex[3], ey[3], len[3];
+  float ex[3], ey[3], len[3], longest = 0.f;
   for (int i = 0; i < 3; ++i) {
     const int j = (i + 1) % 3;
     ex[i] = px[j] - px[i];
     ey[i] = py[j] - py[i];
     len[i] = sqrtf(ex[i] * ex[i] + ey[i] * ey[i]);
     if (!(len[i] > 0.f)) return e;
+    longest = fmaxf(longest, len[i]);
   }
-  // the margin
-  const float w[3] = {p0.w, p1.w, p2.w};
-  float err = 0.f, gz = 0.f;
-  for (int i = 0; i < 3; ++i) {
-    uint32_t b;
-    __builtin_memcpy(&b, &w[i], 4);
-    err = fmaxf(err, hi_float(b));
-    gz = fmaxf(gz, lo_float(b));
-  }
-  const float zmin = fminf(pz[0], fminf(pz[1], pz[2])), zmax = fmaxf(pz[0], fmaxf(pz[1], pz[2]));
-  const float q = lo_float(shape), qz = q * zmax * approx_rcp(zmin), longest = fmaxf(len[0], fmaxf(len[1], len[2]));
-  float bound = err + hi_float(shape) * gz + 38.f * kUnit * pm;
-  if (!(fabsf(area2) >= 16.f * err * longest)) bound += 14.f * kUnit * qz * longest;
-  if (!(qz <= 1e5f) || !(bound <= 1e5f)) return e;
-  const float margin = fmaxf(kEdgeMargin, bound);
+  const float area_unit = kUnit * longest * longest;      // 8 of these bound the area's rounding
+  if (!(fabsf(area2) >= 12.f * area_unit)) return e;
   const float s = area2 > 0.f ? 1.f : -1.f;
   for (int i = 0; i < 3; ++i) {
     // signed distance of (x, y) to edge i, positive inside: s * cross(e, p - p_i) / |e|
     e.a[i] = -s * ey[i] / len[i];
     e.b[i] = s * ex[i] / len[i];
-    e.c[i] = -(e.a[i] * px[i] + e.b[i] * py[i]) + margin;
+    e.c[i] = -(e.a[i] * px[i] + e.b[i] * py[i]);
   }
+  // the margin: what each vertex adds, the largest of them, and the sum of each times the edge opposite
+  const float w[3] = {p0.w, p1.w, p2.w};
+  float err[3], most = 0.f, turn = 0.f;
+  for (int i = 0; i < 3; ++i) {
+    uint32_t b;
+    __builtin_memcpy(&b, &w[i], 4);
+    err[i] = hi_float(b) + hi_float(shape) * lo_float(b);
+    most = fmaxf(most, err[i]);
+    turn += err[i] * len[(i + 1) % 3];
+  }
+  const float rz = approx_rcp(fminf(pz[0], fminf(pz[1], pz[2])));
+  const float q = lo_float(shape), qz = q * fmaxf(pz[0], fmaxf(pz[1], pz[2])) * rz;
+  const float edges = 38.f * kUnit * pm;
+  float bound = most + edges;
+  if (!(turn + 100.f * area_unit <= 0.125f * fabsf(area2))) {
+    bound += 14.f * kUnit * qz * longest;
+  } else if (bound > kEdgeMargin) {
+    // a vertex's error counts by its barycentric over the box
+    const float x[2] = {box.x0 + 0.5f, box.x1 + 0.5f}, y[2] = {box.y0 + 0.5f, box.y1 + 0.5f};
+    const float ra = approx_rcp(fabsf(area2));
+    float sum = 0.f;
+    for (int i = 0; i < 3; ++i) {
+      const int j = (i + 1) % 3;           // the edge opposite
+      const float d = e.c[j] + fmaxf(e.a[j] * x[0], e.a[j] * x[1]) + fmaxf(e.b[j] * y[0], e.b[j] * y[1]);
+      sum += err[i] * (fminf(fmaxf(d, 0.f) * len[j] * ra, 1.25f) + 11.f * kUnit * q * pz[i] * rz);
+    }
+    bound = fminf(bound, 1.4f * sum + 1.25f * edges);
+  }
+  if (!(qz <= 1e5f) || !(bound <= 1e5f)) return e;
+  const float margin = fmaxf(kEdgeMargin, bound);
+  for (int i = 0; i < 3; ++i) e.c[i] += margin;
   e.on = true;
   return e;
 }
+
+// The same of a face without errors of its own (kEdgeMargin alone).
+GVV_HD EdgeTest edge_test(float4 p0, float4 p1, float4 p2) { return edge_test(p0, p1, p2, 0u, Box{0, 0, 0, 0}); }
 
 // The pre-test walked along the rows of a box: the three edge values at the current pixel are
 // kept and advanced by a (one pixel along a row) or, at a row end, by b - (bw - 1) a (back to

@@ -88,7 +88,7 @@ __global__ void __launch_bounds__(256) k_bin(const int32_t* __restrict__ faces, 
         to_queue = true;
         n = 0;
       } else {
-        et = edge_test(p0, p1, p2, tris[(size_t)(bc / C) * F + f].shape);
+        et = edge_test(p0, p1, p2, tris[(size_t)(bc / C) * F + f].shape, bx);
         k = next_tile(et, 0, n, tw, tx0, ty0, W, H, tm.sx, tm.sy);
       }
     }
@@ -224,7 +224,7 @@ __global__ void __launch_bounds__(256) k_tile(TileArgs a) {
           s.z0 = p0.z; s.z1 = p1.z; s.z2 = p2.z;
           s.f = f;
           st[lane] = s;
-          et = edge_test(p0, p1, p2, s.t.shape);
+          et = edge_test(p0, p1, p2, s.t.shape, bx);
         } else {
           bw = bh = 0;
         }

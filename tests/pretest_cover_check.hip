@@ -6,12 +6,14 @@
 // of the span (or, where the span is empty, around the place where the edges are nearest), outside
 // it only.  Per class: the accepted pixels outside the spans (missed) and outside the three half-planes
 // of the direct test (missed_px), the same with kEdgeMargin alone (plain), the faces with the pre-test
-// on, and the largest share of a face's bound that an accepted pixel needed.  Host only.
+// on, the largest share of a face's margin that an accepted pixel needed, and the median margin in px.
+// Host only.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <random>
+#include <vector>
 #include "../gvv-differentiable-cuda-renderer_amd/csrc/gvv_raster.hpp"
 using namespace gvv;
 
@@ -26,6 +28,7 @@ int main(int argc, char** argv) {
     auto logu = [&](double a, double b) { return a * std::pow(b / a, U(rng)); };
     long long missed = 0, missed_px = 0, plain = 0, on = 0, faces = 0, accepted = 0;
     double share = 0;
+    std::vector<double> margins;
     for (int t = 0; t < n; ++t) {
       int W = 1024, H = t % 3 ? 1024 : 389;
       double f = 1.2 * W;
@@ -96,7 +99,7 @@ int main(int argc, char** argv) {
       const int bw = bx.x1 - bx.x0 + 1, bh = bx.y1 - bx.y0 + 1;
       ++faces;
       const TriSetup ts = tri_setup(v[0], v[1], v[2]);
-      const EdgeTest et = edge_test(p[0], p[1], p[2], face_shape(ts));
+      const EdgeTest et = edge_test(p[0], p[1], p[2], face_shape(ts), bx);
       // the three edges without a margin, in binary64
       const EdgeTest ep = edge_test(p_plain[0], p_plain[1], p_plain[2]);
       if (et.on) ++on;
@@ -107,6 +110,7 @@ int main(int argc, char** argv) {
         ed[i][1] = ep.b[i];
         ed[i][2] = -((double)ep.a[i] * p[i].x + (double)ep.b[i] * p[i].y);
       }
+      if (et.on) margins.push_back((double)et.c[0] - ed[0][2]);
       const double bound = et.on ? (double)et.c[0] - ed[0][2] : 1e30;      // this face's margin
       BoxLines bl;
       bl.start(et, bx.x0, bx.y0, bw, bh);
@@ -142,8 +146,9 @@ int main(int argc, char** argv) {
           }
       }
     }
-    printf("%s faces %lld on %lld accepted %lld missed %lld missed_px %lld plain %lld share %.3f\n", names[cls], faces, on, accepted,
-           missed, missed_px, plain, share);
+    std::sort(margins.begin(), margins.end());
+    printf("%s faces %lld on %lld accepted %lld missed %lld missed_px %lld plain %lld share %.3f median %.4f\n", names[cls], faces,
+           on, accepted, missed, missed_px, plain, share, margins[margins.size() / 2]);
   }
   return 0;
 }
