@@ -674,14 +674,18 @@ int launch(ConvArgs a, hipStream_t s, const char* what) {
   return hip_status(what);
 }
 
-// Tile choice: the largest tile that still gives the chip's 256 CUs a workgroup each, as a larger
-// tile reads its operands fewer times.  With 1024 tiles and more, one wave per tile fills the chip
-// and passes no accumulators (backward data of the 64-channel layer at 16 images: 29 us against 38
-// with four waves, of the 128-channel layer 24 against 28); with fewer, the stretches of the
-// reduction are loaded side by side, all at once where the waves' registers hold them (the 4096-deep
+// Tile choice: the largest tile that still gives the chip's 1024 SIMDs a wave each, as a larger
+// tile reads its operands fewer times, or failing that its 256 CUs a workgroup each.  With 1024 tiles
+// and more, one wave per tile fills the chip and passes no accumulators (backward data of the
+// 64-channel layer at 16 images: 29 us against 38 with four waves, of the 128-channel layer 24 against
+// 28); 64 x 128 tiles, where there are so many, take 58 us against 70 with 64 x 64 (128 -> 128 channels,
+// 3 x 3, stride 1, 4 x 128^2; staged through LDS 65) and 105 against 134 (256 -> 256, 8 x 64^2; 146), but
+// 44 against 41 over a reduction of 9 steps (32 -> 64, stride 2, 64 x 128^2), where the output counts.  With
+// fewer, the stretches of the reduction are loaded side by side: 64 x 64 tiles by two waves, as with four
+// the accumulators travel twice as far (64 -> 64, 3 x 3, stride 1, 16 x 56^2: 21 us, 28 with four waves,
+// staged through LDS 22; the 64 -> 128 layer of 16 images 14.4 against 15.4); smaller tiles all at once where the waves' registers hold them (the 4096-deep
 // head of one image: 13 us with 16 waves, 21 with 8 and two rounds of loads, 75 with one wave; the
-// 2304-deep layer 9.4 us with 8 waves, 11.8 with 16, whose accumulators travel twice as far).  Tiles
-// of 32 x 128 and 64 x 128 were no faster (30 and 30 us for those two).
+// 2304-deep layer 9.4 us with 8 waves, 11.8 with 16, whose accumulators travel twice as far).
 template <bool FWD>
 int launch_conv(const ConvArgs& a, hipStream_t s, const char* what) {
   const ConvGeom& g = a.g;
@@ -692,8 +696,9 @@ int launch_conv(const ConvArgs& a, hipStream_t s, const char* what) {
   auto tiles = [&](int bp, int bq) { return ((P + bp - 1) / bp) * ((Q + bq - 1) / bq); };
   if (P <= 32 && tiles(32, 64) >= 1024) return launch<FWD, 2, 4, 1, 2>(a, s, what);
   if (P <= 32 && tiles(32, 64) >= 256) return launch<FWD, 2, 4, 4, 3>(a, s, what);
+  if (P > 32 && steps >= 16 && tiles(64, 128) >= 1024) return launch<FWD, 4, 8, 1, 2>(a, s, what);
   if (P > 32 && tiles(64, 64) >= 1024) return launch<FWD, 4, 4, 1, 2>(a, s, what);
-  if (P > 32 && tiles(64, 64) >= 256) return launch<FWD, 4, 4, 4, 3>(a, s, what);
+  if (P > 32 && tiles(64, 64) >= 256) return launch<FWD, 4, 4, 2, 3>(a, s, what);
   if (P > 16 && tiles(32, 32) >= 256) return launch<FWD, 2, 2, 8, 5>(a, s, what);
   if (steps < 16) return launch<FWD, 1, 1, 4, 4>(a, s, what);
   return steps <= 80 ? launch<FWD, 1, 1, 8, 10>(a, s, what) : launch<FWD, 1, 1, 16, 8>(a, s, what);
