@@ -322,11 +322,12 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
   // face slots: 96, or with the colour terms 82, which leave room for four wavefronts per SIMD in the
   // 160 KB of LDS (200k vertex-coloured faces over 16 x 1024^2, forward + backward 1468 -> 1432 us,
   // 1445 with 88 and 92).  Fewer than 96 of 18 terms gain nothing (fit_batch of 16 x 4 x 512^2, 70k
-  // faces: 1663 us, with 88, 80 and 72 slots 1665, 1668 and 1674).
-  constexpr int kSlots = NT > 18 ? 82 : 96;
+  // faces: 1663 us, with 88, 80 and 72 slots 1665, 1668 and 1674).  A 32 px tile has more faces and is
+  // flushed more often with fewer slots (100k faces over 4 x 1024^2, backward 356 us with 82, 318 with 96).
+  constexpr int kSlots = NT > 18 && TILE < 32 ? 82 : 96;
   __shared__ float s_acc[kSlots][NT1];
   __shared__ int s_face[kSlots];
-  constexpr int kMergeSlots = NT <= 18 ? 32 : 0;     // flush: slots up to which their corners are merged
+  constexpr int kMergeSlots = NT <= 9 ? 16 : NT <= 18 ? 32 : 0;     // flush: slots up to which their corners are merged
   __shared__ int s_vid[kMergeSlots ? 3 * kMergeSlots : 1];   // flush: the corners' vertices, -1 once summed into another corner
   __shared__ int s_list[kMergeSlots ? 64 : 1];       // flush: corners left of a batch of 64
   // face id -> slot: open addressing with linear probing, keys face + 1 (0: free)
@@ -381,8 +382,9 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
   // key words of the face table; gvv_claim.hpp), the corners whose entry names another
   // corner of their vertex add their terms to that one's, and the rest (claimants, and vertices whose
   // entry another vertex took) are flushed, one row of terms per vertex on adjacent lanes.
-  // The LDS additions grow with the faces and the colour terms, so tiles of more than 32 faces, and the
-  // kernel with colour terms, flush slot by slot: forward + backward 632 -> 625 us at 100k textured
+  // The LDS additions grow with the faces and the colour terms, so tiles of more than 32 faces (16 with 9
+  // terms a face, whose requests are fewer: backward 82 us at 100k faces over 4 x 1024^2, 86 with 32, 45
+  // either way at 2k faces), and the kernel with colour terms, flush slot by slot: forward + backward 632 -> 625 us at 100k textured
   // faces over 8 x 1024^2 (about 34 faces a tile), 276 -> 253 us at 320 faces over 4 x 1024^2 (where
   // every tile adds to the same few vertices), 159 -> 156 us at 16k faces over 6 x 333 x 477; merging
   // every tile takes 1780 us for 1663 at 16 x 4 x 512^2 with 70k faces.
@@ -461,8 +463,17 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
   int nidf = round_pixel(0, npx, npy, nidx);
   int ni0 = 0, ni1 = 0, ni2 = 0;
   if (nidf >= 0) { ni0 = a.faces[3 * nidf]; ni1 = a.faces[3 * nidf + 1]; ni2 = a.faces[3 * nidf + 2]; }
-  for (int round = 0;; ++round) {
-    const bool last = round == RT * RT;       // after the rounds: flush only
+  // With 18 terms the flush has one place in the loop over the rounds, where a round finds too few slots
+  // and once more after the last round: a second copy behind the loop costs registers (100k textured
+  // faces over 4 x 1024^2 with the model-to-data term, 260 us against 244).  Elsewhere the loop is the
+  // rounds alone: with one round (8 px tiles) the extra turn took 128 registers for 78 and spilled (2k
+  // faces 272 us against 199), with 27 terms 232 against 228 in 32 px tiles.  The loop of 16 px tiles
+  // without per-face terms is unrolled: 100k textured faces over 4 x 1024^2, 84 us rolled, 70 unrolled.
+  constexpr bool kLoopFlush = RT > 1 && NT == 18;
+  constexpr int kUnroll = NT == 0 && RT == 2 ? 4 : 1;
+#pragma unroll kUnroll
+  for (int round = 0; kLoopFlush || round < RT * RT; ++round) {
+    const bool last = kLoopFlush && round == RT * RT;       // after the rounds: flush only
     const int px = npx, py = npy, idf = last ? -1 : nidf, i0 = ni0, i1 = ni1, i2 = ni2;
     const size_t idx = nidx;
     if (round + 1 < RT * RT) nidf = round_pixel(round + 1, npx, npy, nidx);
@@ -508,16 +519,13 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
       }
       __syncthreads();
     }
-    if (NT == 0) {
-      if (last) break;
-      continue;
-    }
+    if (NT == 0) continue;
     // assign each distinct face of this round a slot (reusing slots of earlier rounds).  The
     // round adds at most as many faces as it has runs of equal ids along the lanes (a run
     // starts where a lane's face differs from the previous lane's, or at a 16-lane row start),
     // so flushing first when fewer slots remain keeps every slot of this round valid until its
     // terms are added, without flushing a tile whose faces all fit
-    {
+    if (RT > 1) {
       const int prev = __builtin_amdgcn_update_dpp(-2, idf, 0x111, 0xf, 0xf, false);   // row_shr:1
       const int runs = __popcll(__ballot(idf >= 0 && idf != prev));
       if (nslots > 0 && (last || nslots + runs > kSlots)) flush();
@@ -563,6 +571,7 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
         if (t[k] != 0.f) atomicAdd(&s_acc[myslot][k], t[k]);
     }
   }
+  if (NT > 0 && !kLoopFlush && nslots > 0) flush();
   if (SHADED) {
     // lane 2k stores the tile's total of coefficient k
     const float s = any ? wave_sums27(sh_acc, lane) : 0.f;
