@@ -164,7 +164,7 @@ __device__ __forceinline__ void pixel_terms(const BackwardArgs& a, const Camera&
   const V3 d = pixel_ray(cam, px + 0.5f, py + 0.5f);
   V3 abc;
   if (HAVE_BARY) abc = v3(ba, bb, 1.f - ba - bb);
-  else abc = ray_barycentric(ts, cam_origin_scaled(cam), d);
+  else abc = SHADED ? ray_barycentric(ts, cam_origin_scaled(cam), d) : ray_barycentric_div(ts, cam_origin_scaled(cam), d);
   const float w3[3] = {abc.x, abc.y, abc.z};
   // textured: the four texels of the backward's blend (Grad.cu:282-312; not the forward's
   // nearest texel) are loaded before the normal and the illumination are formed, which do not
