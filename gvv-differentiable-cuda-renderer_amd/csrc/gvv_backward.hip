@@ -375,7 +375,7 @@ __device__ __forceinline__ void pixel_grad_body(const BackwardArgs& a, int64_t w
 
   // Flush of the slots by lane-parallel global atomics.  Atomics are executed on the memory side, at 16
   // to 20 G requests/s whatever the scope, and this kernel came to 17 G/s (5.0 M in 294 us at 100k
-  // textured faces over 8 x 1024^2; 3.6 M in 284 us now, where the VALU is the bound at 73%), so where
+  // textured faces over 8 x 1024^2; 3.6 M in 284 to 303 us now, where the VALU is the bound at 69 to 73%), so where
   // it is cheap the requests are reduced first: a vertex
   // of the tile belongs to several of its faces (six in a regular mesh), and the slots' corners of one
   // vertex are summed in LDS.  Every corner writes itself to its vertex's entry of a claim table (the

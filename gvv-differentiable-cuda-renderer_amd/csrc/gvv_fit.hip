@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(kThreads) k_masked_sq_grad(const float* __rest
 
 // ---- shape model -------------------------------------------------------------------------
 constexpr int kShapeSubjects = 16;     // subjects per backward workgroup (grid.y covers more)
-constexpr int kShapeMaxSubjects = 65535 * 4;   // the forward's grid.y limit at 4 subjects per thread
+constexpr int kShapeMaxSubjects = 65535 * 4;   // what the entry points take (the forward's grid.y reaches 65535 groups of 16)
 constexpr int kShapeChunk = 64;        // vertices per backward workgroup
 constexpr int kShapeRow = 3 * kShapeChunk + 4;   // padded LDS row: 16-byte reads of 16 rows spread over the banks
 constexpr int kShapeWaves = 4;         // waves of a backward workgroup, each with a quarter of the chunk

@@ -393,9 +393,9 @@ __device__ __forceinline__ void append_spans(unsigned* cand, int& count, int rem
 // lanes write their spans there; a full list (always a multiple of 64) is tested and emptied.
 // The spans replace an edge test of every box pixel, one pixel of 64 boxes per step with 13.75 of
 // the 64 lanes passing on average at 100k triangles over 8 x 1024^2 views: 249 -> 153 us there.
-// What bounds it now, there, is the memory side's rate of atomic requests: 2.59 M in 137 us, 19 G/s
-// of the 21 G/s that scattered atomics reach (the large-face pass the same, 0.72 M in 38 us), with
-// VALU issue at 60% (51 M instructions).  Reading a pixel's key before the exact test, to skip the
+// What bounds it now, there, is the memory side's rate of atomic requests, 2.24 M in 113 us, 20 G/s
+// of the 21 G/s that scattered atomics reach (the large-face pass 0.50 M in 31 us, 16 G/s), and
+// VALU issue at 83% (57 M instructions).  Reading a pixel's key before the exact test, to skip the
 // atomic where the face cannot win, adds a memory-side request for each it saves: 165 us.
 // Appends the lanes' faces with `large` set to the large-face queue, with one atomic per wavefront.
 __device__ __forceinline__ void queue_large(const RasterArgs& ra, bool large, int bc, int f) {

@@ -35,7 +35,7 @@ GVV_HD V3 cross(V3 a, V3 b) { return v3(a.y * b.z - a.z * b.y, a.z * b.x - a.x *
 // 1 / sqrt, against 4.8 for an FMA.  On the host they are the IEEE operations themselves.
 //   rcp_rn       one Newton step on the 1-ulp hardware reciprocal (17 cycles).  Every binary32 x
 //                with 2^-100 <= |x| < 2^100 was compared with 1 / x on the device; others divide.
-//   sqrt_rn      one correction of x rsq(x) (27 cycles), compared likewise for every x in that
+//   sqrt_rn      one Newton correction of x rsq(x) (27 cycles), compared likewise for every x in that
 //                range; others take sqrtf.
 //   quot         a / b from a binary64 reciprocal r of b (recip64, within 2^-52 of 1 / b): one
 //                binary64 product, rounded to binary32 (14 cycles).  The quotient of two 24-bit

@@ -240,7 +240,8 @@ GVV_HD EdgeTest edge_test(float4 p0, float4 p1, float4 p2) { return edge_test(p0
 // the row's first pixel, one row down), instead of being evaluated anew at every pixel.  The
 // stepped values differ from the direct ones by rounding only (at most 64 steps of values
 // under 100 px), far inside the margin; tests/edge_margin_check.hip runs this walk over every
-// box it draws and counts the accepted pixels that it would reject (none).
+// box it draws and counts the accepted pixels that it would reject (none).  The depth pass has
+// walked lines (BoxLines) since; only that check uses this walk.
 struct EdgeWalk {
   float e[3];     // edge values at the current pixel
   float w[3];     // row-end step b - (bw - 1) a
@@ -309,7 +310,8 @@ struct BoxLines {
 // Conservative x-range [xl, xr] of bounding-box row y (pixel centres at y + 0.5) inside the
 // three half-planes of the edge pre-test, widened by one pixel on each side so that float
 // rounding of the bounds never drops a pixel the pre-test would pass.  Without a usable edge
-// test the whole row is returned.
+// test the whole row is returned.  The kernels take BoxLines' spans; tests/raster_span_check.hip
+// alone uses this.
 GVV_HD void row_span(const EdgeTest& e, int y, int x0, int x1, int& xl, int& xr) {
   xl = x0;
   xr = x1;
